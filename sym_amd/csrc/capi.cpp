@@ -361,7 +361,7 @@ int relx_bound_query(const relx_bound *bound, relx_bound_info *out) {
       const std::vector<relx::KArgs> ls = relx::axis_launches(dp, -1, 0, 0);
       int tiles = 0, rows = 0;
       for (const relx::KArgs &a : ls)
-        if (!a.edge_box) {
+        if (a.family == relx::kFamTranspose) {
           ++tiles;
           rows += (a.t_flags & relx::kTileRowChannel) ? 1 : 0;
         }

@@ -388,9 +388,17 @@ __device__ __forceinline__ void pack(const uint32_t (&v)[V], vec4 *out) {
   }
 }
 
+// Parameter entry of element e of a vector with one channel per element. A
+// cut vector (CUT: its last elements lie past the end of its row and are not
+// stored) stays inside the table.
+template <bool CUT>
+__device__ __forceinline__ uint32_t chan_elem(const DevStage &s, uint32_t c, uint32_t e) {
+  return CUT ? min(c + e, s.ch_re_div.d - 1) : c + e;
+}
+
 // One stage over V consecutive destination elements starting at dense result
 // offset `o` (channel constant or +1 per element, proven on the host).
-template <int V>
+template <int V, bool CUT = false>
 __device__ __forceinline__ void stage_vec(const KArgs &a, const DevStage &s, uint32_t (&v)[V],
                                           int64_t o) {
   const uint32_t c = chan_of(s, o);
@@ -424,7 +432,7 @@ __device__ __forceinline__ void stage_vec(const KArgs &a, const DevStage &s, uin
     } else {
 #pragma unroll
       for (int e = 0; e < V; ++e)
-        v[e] = op_quant(v[e], a.pf[s.scale_off + c + e]);
+        v[e] = op_quant(v[e], a.pf[s.scale_off + chan_elem<CUT>(s, c, e)]);
     }
     break;
   default:
@@ -437,15 +445,15 @@ __device__ __forceinline__ void stage_vec(const KArgs &a, const DevStage &s, uin
     } else {
 #pragma unroll
       for (int e = 0; e < V; ++e)
-        v[e] = op_dequant(v[e], a.pf[s.scale_off + c + e],
-                          a.pi[s.zp_off + (s.zp_per_ch ? c + e : 0u)]);
+        v[e] = op_dequant(v[e], a.pf[s.scale_off + chan_elem<CUT>(s, c, e)],
+                          a.pi[s.zp_off + (s.zp_per_ch ? chan_elem<CUT>(s, c, e) : 0u)]);
     }
   }
 }
 
 // The stage chain over one vector: compile-time bodies for the common
 // sequences, per-stage dispatch (stage index still compile-time) otherwise.
-template <int CH, int V>
+template <int CH, int V, bool CUT = false>
 __device__ __forceinline__ void chain_vec(const KArgs &a, uint32_t (&v)[V], int64_t o) {
   if constexpr (CH == kChainNone) {
   } else if constexpr (CH == kChainF32F16) {
@@ -468,11 +476,11 @@ __device__ __forceinline__ void chain_vec(const KArgs &a, uint32_t (&v)[V], int6
     } else {
 #pragma unroll
       for (int e = 0; e < V; ++e)
-        v[e] = op_f32_f16(op_dequant(v[e], a.pf[s.scale_off + c + e],
-                                     a.pi[s.zp_off + (s.zp_per_ch ? c + e : 0u)]));
+        v[e] = op_f32_f16(op_dequant(v[e], a.pf[s.scale_off + chan_elem<CUT>(s, c, e)],
+                                     a.pi[s.zp_off + (s.zp_per_ch ? chan_elem<CUT>(s, c, e) : 0u)]));
     }
   } else if constexpr (CH == kChainDeq) {
-    stage_vec<V>(a, a.chain.st[0], v, o);
+    stage_vec<V, CUT>(a, a.chain.st[0], v, o);
   } else if constexpr (CH == kChainF16Quant) {
     const DevStage &s = a.chain.st[1];
     const uint32_t c = chan_of(s, o);
@@ -484,16 +492,16 @@ __device__ __forceinline__ void chain_vec(const KArgs &a, uint32_t (&v)[V], int6
     } else {
 #pragma unroll
       for (int e = 0; e < V; ++e)
-        v[e] = quant_value(op_f16_f32_value(v[e]), a.pf[s.scale_off + c + e]);
+        v[e] = quant_value(op_f16_f32_value(v[e]), a.pf[s.scale_off + chan_elem<CUT>(s, c, e)]);
     }
   } else if constexpr (CH == kChainQuant) {
-    stage_vec<V>(a, a.chain.st[0], v, o);
+    stage_vec<V, CUT>(a, a.chain.st[0], v, o);
   } else {
 #pragma unroll
     for (int k = 0; k < kMaxStages; ++k) {
       if (k >= a.chain.n)
         break;
-      stage_vec<V>(a, a.chain.st[k], v, o);
+      stage_vec<V, CUT>(a, a.chain.st[k], v, o);
     }
   }
 }
@@ -525,7 +533,7 @@ template <int CH> __device__ __forceinline__ VecParams fetch_params(const KArgs 
 }
 
 // chain_vec with the parameters of a channel-constant vector given.
-template <int CH, int V>
+template <int CH, int V, bool CUT = false>
 __device__ __forceinline__ void chain_vec_p(const KArgs &a, uint32_t (&v)[V], int64_t o,
                                             const VecParams &p) {
   if constexpr (CH == kChainDeqF16) {
@@ -543,7 +551,79 @@ __device__ __forceinline__ void chain_vec_p(const KArgs &a, uint32_t (&v)[V], in
       return;
     }
   }
-  chain_vec<CH, V>(a, v, o);
+  chain_vec<CH, V, CUT>(a, v, o);
+}
+
+// ------------------------------------------------------ unaligned accesses
+
+// gfx950 global accesses take any byte address: 16 bytes at whatever
+// alignment a row gives them.
+typedef uint32_t vec4u __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t vec2u __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t word_u __attribute__((aligned(1)));
+typedef uint16_t half_u __attribute__((aligned(1)));
+
+template <int NB, bool NT = false> __device__ __forceinline__ vec4 ldu_n(const uint8_t *p) {
+  vec4 r = {0u, 0u, 0u, 0u};
+  if constexpr (NB == 16) {
+    const vec4u *q = reinterpret_cast<const vec4u *>(p);
+    r = NT ? __builtin_nontemporal_load(q) : *q;
+  } else if constexpr (NB == 8) {
+    const vec2u *q = reinterpret_cast<const vec2u *>(p);
+    const vec2 t = NT ? __builtin_nontemporal_load(q) : *q;
+    r.x = t.x;
+    r.y = t.y;
+  } else {
+    static_assert(NB == 4, "4, 8 or 16 bytes");
+    const word_u *q = reinterpret_cast<const word_u *>(p);
+    r.x = NT ? __builtin_nontemporal_load(q) : *q;
+  }
+  return r;
+}
+
+template <int NB, bool NT = false> __device__ __forceinline__ void stu_n(uint8_t *p, const vec4 &v) {
+  if constexpr (NB == 16) {
+    vec4u *q = reinterpret_cast<vec4u *>(p);
+    if constexpr (NT)
+      __builtin_nontemporal_store(v, q);
+    else
+      *q = v;
+  } else if constexpr (NB == 8) {
+    vec2u *q = reinterpret_cast<vec2u *>(p);
+    const vec2 t = {v.x, v.y};
+    if constexpr (NT)
+      __builtin_nontemporal_store(t, q);
+    else
+      *q = t;
+  } else {
+    word_u *q = reinterpret_cast<word_u *>(p);
+    if constexpr (NT)
+      __builtin_nontemporal_store(v.x, q);
+    else
+      *q = v.x;
+  }
+}
+
+// The first n < 16 bytes of v: at most one store each of 8, 4, 2 and 1 bytes.
+__device__ __forceinline__ void stu_cut(uint8_t *p, vec4 v, uint32_t n) {
+  if (n & 8) {
+    *reinterpret_cast<vec2u *>(p) = vec2{v.x, v.y};
+    v.x = v.z;
+    v.y = v.w;
+    p += 8;
+  }
+  if (n & 4) {
+    *reinterpret_cast<word_u *>(p) = v.x;
+    v.x = v.y;
+    p += 4;
+  }
+  if (n & 2) {
+    *reinterpret_cast<half_u *>(p) = static_cast<uint16_t>(v.x);
+    v.x >>= 16;
+    p += 2;
+  }
+  if (n & 1)
+    *p = static_cast<uint8_t>(v.x);
 }
 
 // ---------------------------------------------------------------- stream
@@ -1530,6 +1610,8 @@ hipError_t stream_fast(const KArgs &a, hipStream_t s, bool &handled);
 hipError_t stream_generic(const KArgs &a, hipStream_t s);
 hipError_t transpose_fast(const KArgs &a, hipStream_t s, bool &handled);
 hipError_t transpose_generic(const KArgs &a, hipStream_t s);
+hipError_t transpose_ragged_fast(const KArgs &a, hipStream_t s, bool &handled);
+hipError_t transpose_ragged_generic(const KArgs &a, hipStream_t s);
 hipError_t interleave_fast(const KArgs &a, hipStream_t s, bool &handled);
 hipError_t interleave_generic(const KArgs &a, hipStream_t s);
 hipError_t permute_fast(const KArgs &a, hipStream_t s, bool &handled);

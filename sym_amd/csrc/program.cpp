@@ -271,6 +271,74 @@ int vec_mode(const HostStage &s, const Prepared &p, const Bound &b, int64_t V) {
   return -1;
 }
 
+// Channel behaviour along a destination row of `len` elements (the innermost
+// coalesced axis, whose rows start at multiples of len): 0 constant along the
+// row, 1 the column itself, -1 neither.
+int row_mode(const HostStage &s, const Prepared &p, const Bound &b, int64_t len) {
+  if (s.mode == kChanNone)
+    return 0;
+  if (s.mode != kChanDim)
+    return -1;
+  const int64_t rs = p.res_strides[static_cast<size_t>(s.dim)];
+  const int64_t re = b.result_extents[static_cast<size_t>(s.dim)];
+  if (re > s.len)
+    return -1;
+  if (rs % len == 0)
+    return 0;
+  if (rs == 1 && re == len)
+    return 1;
+  return -1;
+}
+
+bool transpose_family(int family) {
+  return family == kFamTranspose || family == kFamRaggedTranspose;
+}
+
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Bytes above which a launch's lines do not stay in the 256 MB Infinity Cache
+// until the next launch on other buffers: its rows then come from HBM.
+constexpr int64_t kColdBytes = int64_t{96} << 20;
+
+// Tile widths, order and cache policy of a ragged transpose launch that moves
+// `bytes`. A row that starts inside a line shares it with the next tile.
+//   Destination rows that start on 64-byte boundaries: streaming stores of
+//   64 x 64 tiles (int8 [4096,11007] -> f16 24.5 us against 34.8 cached).
+//   Others are written in part by two tiles, which streaming would send to
+//   memory as two partial writes (f32 [16,1001,770] -> f16 16.5 against 13.0
+//   us cached). Cold launches take large tiles, which have fewer such lines,
+//   and streaming loads (f32 [32,2047,513] -> f16, 202 MB, 39.9 us against
+//   49.3 us with 64 x 64 tiles and cached loads); launches that fit the
+//   Infinity Cache take 64 x 64 tiles, of which more run at once (int8
+//   [1027,4099] -> f32, 21 MB, 8.6 against 14.2 us) with cached loads (f32
+//   [16,1001,770] -> f16 13.0 against 15.6 us streaming).
+// Each XCD takes a contiguous run of tiles (74 MB activation above: 18.6 ->
+// 13.0 us), so tiles that share a line meet in one L2, except where no line
+// is shared: words whose rows are all aligned (f32 [262000,64] 22.9 -> 21.0
+// us without).
+void ragged_policy(KArgs &a, int64_t bytes) {
+  auto aligned = [&](int64_t base, int64_t stride, int64_t batch, int w) {
+    return (base * w) % 64 == 0 && (stride * w) % 64 == 0 && (batch * w) % 64 == 0;
+  };
+  bool src = true, dst = true;
+  for (int j = 0; j < kBatchLevels; ++j) {
+    src = src && aligned(a.sbase, a.t_ssc, a.lv[j].ss, a.win);
+    dst = dst && aligned(a.dbase, a.t_dsq, a.lv[j].ds, a.wout);
+  }
+  const bool cold = bytes >= kColdBytes, xcd = a.win == 1 || !src || !dst;
+  const bool large = !dst && cold;
+  a.t_wq = static_cast<uint16_t>(large ? ragged_large_q(a.win) : kRaggedTile);
+  a.t_wc = static_cast<uint16_t>(large ? kRaggedLargeC : kRaggedTile);
+  a.t_flags = (xcd ? kTileXcd : 0u) | (cold && xcd ? kTileNtLoad : 0u) | (dst ? kTileNtStore : 0u);
+}
+
+// Aligned boxes of at least this many elements whose last tiles are cut run
+// as one ragged launch.
+constexpr int64_t kRaggedWholeElements = int64_t{1} << 14;
+
+// Shortest q and c extents that take the ragged transpose's tiles.
+constexpr int64_t kRaggedMinExtent = 16;
+
 } // namespace
 
 std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, uint32_t k) {
@@ -417,6 +485,18 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
     }
     return true;
   };
+  // the same for kernels whose vectors start at any element of a row but
+  // never leave it: the channel is constant along a row, or the row's column
+  const int64_t row_len = r > 0 ? pext[static_cast<size_t>(r - 1)] : 1;
+  auto row_channels_ok = [&] {
+    for (uint32_t i = k; i < nst; ++i) {
+      const int m = row_mode(p.stages[i], p, b, row_len);
+      if (m < 0 || (p.stages[i].mode == kChanDim && !off32))
+        return false;
+      ch.st[i - k].vec = static_cast<uint8_t>(m);
+    }
+    return true;
+  };
   // stage sequences with a compile-time kernel body
   int chain_code = kChainGeneric;
   {
@@ -522,6 +602,29 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
         }
       }
     }
+    // ragged transpose: the same axes at any extents and alignments (checked
+    // after the interleave, whose few channels would leave most of a tile
+    // empty)
+    auto ragged_transpose = [&] {
+      if (any_pad || r < 2 || r - 2 > kBatchLevels || a.ss[r - 1] == 1)
+        return false;
+      int qa = -1;
+      for (int i = 0; i < r - 1; ++i)
+        if (a.ss[i] == 1 && a.vext[i] > 1)
+          qa = i;
+      if (qa < 0 || a.vext[qa] < kRaggedMinExtent || a.vext[r - 1] < kRaggedMinExtent)
+        return false;
+      a.t_wq = a.t_wc = kRaggedTile; // boxes start at multiples (large tiles: any start)
+      int64_t tiles = ceil_div(a.vext[qa], a.t_wq) * ceil_div(a.vext[r - 1], a.t_wc);
+      for (int i = 0; i < r - 1; ++i)
+        if (i != qa)
+          tiles *= a.vext[i];
+      if (tiles >= (int64_t{1} << 22) || !row_channels_ok())
+        return false;
+      dp->qa = qa;
+      dp->ca = r - 1;
+      return true;
+    };
     // interleave: [batch..., P, C(pad)] planar source
     if (family == kFamGeneric && r >= 2 && r - 2 <= kBatchLevels && a.ss[r - 1] != 1 &&
         a.ss[r - 2] == 1 && a.ds[r - 2] == pext[static_cast<size_t>(r - 1)]) {
@@ -541,13 +644,15 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
         a.cpad = static_cast<int32_t>(cp);
       }
     }
+    if (family == kFamGeneric && ragged_transpose())
+      family = kFamRaggedTranspose;
   }
   if (family == kFamGeneric)
     for (uint32_t i = k; i < nst; ++i)
       ch.st[i - k].vec = 0;
   dp->family = family;
   a.chain_code = chain_code;
-  static const char *names[] = {"generic", "stream", "transpose", "interleave", "permute"};
+  static const char *names[] = {"generic", "stream", "transpose", "interleave", "permute", "generic"};
   dp->kernel = names[family];
 
   // ------------------------------------------------------- chunk axis
@@ -568,7 +673,7 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
         dp->chunk_stride = a.ss[ax];
         if (family == kFamStream && ax == r - 1)
           dp->chunk_align = V;
-        else if (family == kFamTranspose && (ax == dp->qa || ax == dp->ca))
+        else if (transpose_family(family) && (ax == dp->qa || ax == dp->ca))
           dp->chunk_align = ax == dp->qa ? a.t_wq : a.t_wc;
         else if (family == kFamInterleave && ax == r - 2)
           dp->chunk_align = a.vec;
@@ -604,8 +709,8 @@ int64_t box_work(const DeviceProgram &dp, const Box &b) {
     int64_t e = b.ext[i];
     if (dp.family == kFamStream && i == r - 1)
       e /= a.vec;
-    else if (dp.family == kFamTranspose && (i == dp.qa || i == dp.ca))
-      e /= i == dp.qa ? a.t_wq : a.t_wc;
+    else if (transpose_family(dp.family) && (i == dp.qa || i == dp.ca))
+      e = ceil_div(e, i == dp.qa ? a.t_wq : a.t_wc);
     else if (dp.family == kFamInterleave && i == r - 2)
       e /= a.vec;
     else if (dp.family == kFamInterleave && i == r - 1)
@@ -626,7 +731,7 @@ int64_t split_align(const DeviceProgram &dp, int i) {
   const int r = dp.base.rank;
   if (dp.family == kFamStream && i == r - 1)
     return dp.base.vec;
-  if (dp.family == kFamTranspose && (i == dp.qa || i == dp.ca))
+  if (transpose_family(dp.family) && (i == dp.qa || i == dp.ca))
     return i == dp.qa ? dp.base.t_wq : dp.base.t_wc;
   if (dp.family == kFamInterleave && i == r - 2)
     return dp.base.vec;
@@ -643,7 +748,7 @@ int64_t split_align(const DeviceProgram &dp, int i) {
 // 2-D block of the transpose/interleave kernels).
 bool level_axis(const DeviceProgram &dp, int i) {
   const int r = dp.base.rank;
-  if (dp.family == kFamTranspose)
+  if (transpose_family(dp.family))
     return i != dp.qa && i != dp.ca;
   if (dp.family == kFamInterleave)
     return i < r - 2;
@@ -747,7 +852,7 @@ KArgs edge_args(const DeviceProgram &dp, const Box &b) {
   }
   a.work64 = box_elements(b, a.rank);
   a.work = 0;
-  a.edge_box = 1;
+  a.family = kFamGeneric;
   return a;
 }
 
@@ -824,7 +929,9 @@ bool permute_direct(KArgs &a, int64_t C, int64_t M, int64_t E) {
   return true;
 }
 
-KArgs launch_args(const DeviceProgram &dp, const Box &b) {
+// `family`: the program's own, or kFamRaggedTranspose for a box of a
+// transpose program whose last tiles are cut.
+KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
   KArgs a = dp.base;
   const int r = a.rank;
   for (int i = 0; i < r; ++i) {
@@ -844,9 +951,8 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b) {
   }
   for (int i = 0; i < kMaxRank; ++i)
     a.lv[i] = trivial_level();
-  const int64_t work = box_work(dp, b);
-  a.work = static_cast<uint32_t>(work);
-  a.work64 = work;
+  int64_t work = box_work(dp, b);
+  a.family = family;
   // batch levels of the 2-D families: every axis but skip0/skip1, outer first
   auto batch = [&](int skip0, int skip1) {
     int idx[kMaxRank], n = 0;
@@ -856,7 +962,7 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b) {
     for (int j = 0; j < n; ++j)
       a.lv[kBatchLevels - n + j] = axis_level(a, b, idx[j], 1);
   };
-  switch (dp.family) {
+  switch (family) {
   case kFamStream:
     for (int i = 0; i < r; ++i)
       a.lv[a.nlev - r + i] = axis_level(a, b, i, i == r - 1 ? a.vec : 1);
@@ -891,6 +997,25 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b) {
     a.t_ssc = a.ss[dp.ca];
     a.t_dsq = a.ds[dp.qa];
     break;
+  case kFamRaggedTranspose: {
+    batch(dp.qa, dp.ca);
+    a.t_ssc = a.ss[dp.ca];
+    a.t_dsq = a.ds[dp.qa];
+    ragged_policy(a, box_elements(b, r) * (a.win + a.wout));
+    const int64_t nq = ceil_div(b.ext[dp.qa], a.t_wq), nc = ceil_div(b.ext[dp.ca], a.t_wc);
+    work = box_elements(b, r) / (b.ext[dp.qa] * b.ext[dp.ca]) * nq * nc;
+    const int64_t g = std::min<int64_t>(kTileGroup, nq), full = nq / g * g;
+    a.t_plane = make_div(nq * nc);
+    a.t_group = make_div(g * nc);
+    a.t_g = make_div(g);
+    a.t_tail = make_div(nq - full > 0 ? nq - full : 1);
+    a.t_nc = make_div(nc);
+    a.t_full = static_cast<uint32_t>(full);
+    a.t_choff = 0;
+    a.t_qn = static_cast<uint32_t>(b.ext[dp.qa]);
+    a.t_cn = static_cast<uint32_t>(b.ext[dp.ca]);
+    break;
+  }
   case kFamPermute: {
     int idx[kMaxRank], n = 0;
     for (int i = 0; i < r - 3; ++i)
@@ -916,12 +1041,11 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b) {
     a.i_vc = static_cast<int32_t>(a.vext[r - 1]);
     break;
   default: {
-    int64_t n = 1;
-    for (int i = 0; i < r; ++i)
-      n *= b.ext[i];
-    a.work64 = n;
+    work = box_elements(b, r);
   }
   }
+  a.work = family == kFamGeneric ? 0 : static_cast<uint32_t>(work);
+  a.work64 = work;
   return a;
 }
 
@@ -964,11 +1088,6 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
     b.ext[axis] = phi - plo;
   }
   std::vector<KArgs> out;
-  // A transpose box whose q or c extent is not a multiple of the tile: the
-  // whole tiles go to the tile kernel, the strips past them (the q strip
-  // over the whole c range, the c strip beside the whole q tiles) to the
-  // element-wise kernel. Box starts on those axes are multiples of the tile
-  // (t_wq along q, t_wc along c: chunks and splits keep the tile alignment).
   std::vector<Box> edges;
   if (dp.family == kFamStream && a.rank == 1 && b.ext[0] % a.vec != 0) {
     // the tail of a single contiguous axis (box starts are multiples of V)
@@ -979,36 +1098,45 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
     edges.push_back(e);
     b.ext[0] = m;
   }
-  if (dp.family == kFamTranspose) {
-    const int q = dp.qa, c = dp.ca;
-    const int64_t wq = a.t_wq, wc = a.t_wc;
-    const int64_t mq = b.ext[q] / wq * wq, mc = b.ext[c] / wc * wc;
-    if (mq < b.ext[q]) {
-      Box e = b;
-      e.lo[q] = b.lo[q] + mq;
-      e.ext[q] = b.ext[q] - mq;
-      edges.push_back(e);
+  // A transpose box whose q or c extent is not a multiple of the tile runs
+  // as one ragged launch; a small one keeps its whole tiles on the tile
+  // kernel and runs the strips past them (the q strip over the whole c range,
+  // the c strip beside the whole q tiles) as ragged launches.
+  int family = dp.family;
+  if (family == kFamTranspose && (b.ext[dp.qa] % a.t_wq || b.ext[dp.ca] % a.t_wc)) {
+    if (box_elements(b, a.rank) >= kRaggedWholeElements) {
+      family = kFamRaggedTranspose;
+    } else {
+      const int q = dp.qa, c = dp.ca;
+      const int64_t mq = b.ext[q] / a.t_wq * a.t_wq, mc = b.ext[c] / a.t_wc * a.t_wc;
+      if (mq < b.ext[q]) {
+        Box e = b;
+        e.lo[q] = b.lo[q] + mq;
+        e.ext[q] = b.ext[q] - mq;
+        edges.push_back(e);
+      }
+      if (mc < b.ext[c] && mq > 0) {
+        Box e = b;
+        e.ext[q] = mq;
+        e.lo[c] = b.lo[c] + mc;
+        e.ext[c] = b.ext[c] - mc;
+        edges.push_back(e);
+      }
+      b.ext[q] = mq;
+      b.ext[c] = mc;
     }
-    if (mc < b.ext[c] && mq > 0) {
-      Box e = b;
-      e.ext[q] = mq;
-      e.lo[c] = b.lo[c] + mc;
-      e.ext[c] = b.ext[c] - mc;
-      edges.push_back(e);
-    }
-    b.ext[q] = mq;
-    b.ext[c] = mc;
   }
   std::vector<Box> boxes;
   if (box_elements(b, a.rank) > 0)
     split_box(dp, b, boxes);
   out.reserve(boxes.size() + edges.size());
   for (const Box &x : boxes)
-    if (box_work(dp, x) > 0)
-      out.push_back(launch_args(dp, x));
+    if (box_elements(x, a.rank) > 0)
+      out.push_back(launch_args(dp, x, family));
   for (const Box &x : edges)
     if (box_elements(x, a.rank) > 0)
-      out.push_back(edge_args(dp, x));
+      out.push_back(dp.family == kFamTranspose ? launch_args(dp, x, kFamRaggedTranspose)
+                                               : edge_args(dp, x));
   return out;
 }
 
@@ -1087,11 +1215,11 @@ struct Checker {
 
 void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, int64_t wire_hi) {
   DeviceProgram edge;
-  if (a.edge_box && dp_in.family != kFamGeneric) { // run by the element-wise kernel
+  if (a.family != dp_in.family) { // a launch of another family than the program's
     edge = dp_in;
-    edge.family = kFamGeneric;
+    edge.family = a.family;
   }
-  const DeviceProgram &dp = a.edge_box && dp_in.family != kFamGeneric ? edge : dp_in;
+  const DeviceProgram &dp = a.family != dp_in.family ? edge : dp_in;
   const Checker ck{dp,          a,           wire_hi < 0 ? dp.wire_elems : wire_hi,
                    dp.dst_elems, dp.pf.size(), dp.pi.size(),
                    wire_lo};
@@ -1181,6 +1309,52 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
           if (rowch && chan_of(a.chain.st[0], o) != a.t_choff + static_cast<uint32_t>(q0 + row))
             bad_launch(dp, "a row-indexed launch reads another parameter entry");
         }
+    }
+    break;
+  }
+  case kFamRaggedTranspose: {
+    if (a.work64 > (int64_t{1} << 22) || a.work != a.work64)
+      bad_launch(dp, "more tiles than one launch takes");
+    const int VO = 16 / wout;
+    const int64_t TQ = a.t_wq, TC = a.t_wc, Q = a.t_qn, C = a.t_cn;
+    const int64_t nq = ceil_div(Q, TQ), nc = ceil_div(C, TC);
+    const bool large = TC == kRaggedLargeC;
+    if (TQ != (large ? ragged_large_q(win) : kRaggedTile) || !(large || TC == kRaggedTile) || Q < 1 ||
+        C < 1 || (a.t_flags & ~(kTileXcd | kTileNtLoad | kTileNtStore)) ||
+        (large && (a.t_flags & kTileNtStore)) || a.t_nc.d != nc || int64_t{a.t_plane.d} != nq * nc)
+      bad_launch(dp, "tile geometry disagrees with the kernel");
+    std::vector<bool> seen(a.work, false); // the order must be a bijection
+    for (uint32_t blk = 0; blk < a.work; ++blk) {
+      const uint32_t t = (a.t_flags & kTileXcd) ? xcd_tile(blk, a.work) : blk;
+      if (t >= a.work)
+        bad_launch(dp, "a block maps past the last tile");
+      uint32_t tq, tc, r2;
+      tile_of(a, t, tq, tc, r2);
+      if (tq >= nq || tc >= nc)
+        bad_launch(dp, "tile coordinates outside the plane");
+      const size_t id = (static_cast<size_t>(r2) * nq + tq) * nc + tc;
+      if (id >= seen.size() || seen[id])
+        bad_launch(dp, "the tile order visits a tile twice");
+      seen[id] = true;
+      int64_t sbase = a.sbase, dbase = a.dbase;
+      if (decompose_rt(kBatchLevels, a.lv, r2, sbase, dbase))
+        bad_launch(dp, "a transpose tile reaches a pad");
+      const int64_t q0 = tq * TQ, c0 = tc * TC;
+      const int64_t qn = std::min(TQ, Q - q0), cn = std::min(TC, C - c0);
+      // rows of qn elements; the last vector of a cut row ends with the row
+      // and may start before the tile, inside the same source row (strides
+      // are not negative: the first and last row reach the furthest)
+      const int64_t before = std::max<int64_t>(0, 16 / win - qn);
+      if (a.box_lo[dp.qa] + q0 < before)
+        bad_launch(dp, "a cut vector starts before its row");
+      for (int64_t row : {int64_t{0}, cn - 1})
+        ck.src_run(sbase + (c0 + row) * a.t_ssc + q0 - before, qn + before, false);
+      for (int64_t row = 0; row < qn; ++row) {
+        const int64_t d = dbase + (q0 + row) * a.t_dsq + c0;
+        ck.dst_run(d, cn, false);
+        for (int64_t cv = 0; cv < cn; cv += VO)
+          ck.channels(d + cv, static_cast<int>(std::min<int64_t>(VO, cn - cv)));
+      }
     }
     break;
   }
@@ -1320,24 +1494,20 @@ int64_t launch_all(const DeviceProgram &dp, std::vector<KArgs> launches, const v
                        reinterpret_cast<uintptr_t>(dst) % 16 == 0;
   int64_t n = 0;
   for (KArgs &a : launches) {
-    int family = a.edge_box ? kFamGeneric : dp.family;
-    if (!aligned && family != kFamGeneric) {
-      family = kFamGeneric;
+    if (!aligned && a.family != kFamGeneric && a.family != kFamRaggedTranspose) {
+      a.family = kFamGeneric;
       int64_t e = 1;
       for (int i = 0; i < a.rank; ++i)
         e *= a.box_ext[i];
       a.work64 = e;
     }
-    if (verify_enabled()) {
-      DeviceProgram view = dp;
-      view.family = family;
-      verify_launch(view, a, wire_lo, wire_hi);
-    }
+    if (verify_enabled())
+      verify_launch(dp, a, wire_lo, wire_hi);
     a.src = static_cast<const uint8_t *>(src);
     a.dst = static_cast<uint8_t *>(dst);
     a.pf = pf;
     a.pi = pi;
-    const hipError_t e = launch_box(family, a, status, s);
+    const hipError_t e = launch_box(a.family, a, status, s);
     if (e != hipSuccess)
       fail("backend_failure", std::string("kernel launch: ") + hipGetErrorString(e));
     ++n;

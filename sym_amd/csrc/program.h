@@ -108,7 +108,14 @@ enum Family : int32_t {
   kFamTranspose = 2,  // batched 2-D transpose, LDS tiled
   kFamInterleave = 3, // planar -> interleaved with a small padded inner axis
   kFamPermute = 4,    // swap of two axes above a contiguous inner block, through LDS
+  kFamRaggedTranspose = 5, // batched 2-D transpose of any extents and row alignments
 };
+
+// Tiles of the ragged transpose: 64 q by 64 c, or large ones 128 c wide
+// (one-byte sources 128 q wide too: their tiles are kept in LDS as bytes).
+constexpr int kRaggedTile = 64;
+constexpr int kRaggedLargeC = 128;
+constexpr int ragged_large_q(int win) { return win == 1 ? 128 : 64; }
 
 // Pixels per interleave work item: the packed output of an item fills one
 // 16-byte vector when a pixel is at most 16 bytes, and each plane is read in
@@ -148,6 +155,10 @@ constexpr uint32_t kTileRowChannel = 4;
 // dequantization), so the kernel leaves the subtraction out.
 constexpr uint32_t kTileZeroPoint0 = 8;
 
+// Ragged transposes: streaming loads, streaming stores.
+constexpr uint32_t kTileNtLoad = 16;
+constexpr uint32_t kTileNtStore = 32;
+
 // Decomposition levels of the batch axes of the 2-D families.
 constexpr int kBatchLevels = 3;
 // Work items per launch of a fast kernel, and the source and destination
@@ -185,7 +196,7 @@ struct KArgs {
   // g, tail = the q-tiles of the last, partial group, nc = c-tiles
   FastDiv t_plane, t_group, t_g, t_tail, t_nc;
   uint32_t t_full;  // q-tiles in whole groups
-  uint32_t t_flags; // kTileXcd | kTileSkew | kTileRowChannel
+  uint32_t t_flags; // kTile* flags
   // q-tile width (64, or 128 for one-byte sources) and c-tile width (64, or
   // 128 for one-byte sources with wider results: byte tiles), read on
   // the host only; 16 bits each keep the fields the kernels read where they
@@ -213,6 +224,9 @@ struct KArgs {
   uint32_t p_cmask, p_pad_;
   int64_t p_dsc;        // destination stride of c (M*E)
   Chain chain;
+  // ragged transpose: extents of q and c in the box (the last tile along
+  // either may be cut)
+  uint32_t t_qn, t_cn;
   // ---- generic kernel and host bookkeeping (coalesced destination axes)
   int32_t rank;
   int32_t win, wout; // element bytes of the wire and of the result
@@ -222,8 +236,8 @@ struct KArgs {
   int32_t cpad;      // interleave: padded inner extent
   int32_t vec;       // stream: elements per vector; interleave: pixels per thread
   int32_t res_rank;
-  int32_t edge_box;  // 1: a box of a fast-family program at its unaligned edge,
-                     // run by the generic kernel
+  int32_t family;    // Family of this launch (a program's edge boxes may take
+                     // another one than its whole tiles or vectors)
   int32_t p_direct;  // permute: G*E, E and the run are powers of two, one
                      // batch level, and the parameter stage's channel is c
                      // or 0 (permute_direct)
