@@ -1612,6 +1612,8 @@ hipError_t transpose_fast(const KArgs &a, hipStream_t s, bool &handled);
 hipError_t transpose_generic(const KArgs &a, hipStream_t s);
 hipError_t transpose_ragged_fast(const KArgs &a, hipStream_t s, bool &handled);
 hipError_t transpose_ragged_generic(const KArgs &a, hipStream_t s);
+hipError_t rows_fast(const KArgs &a, hipStream_t s, bool &handled);
+hipError_t rows_generic(const KArgs &a, hipStream_t s);
 hipError_t interleave_fast(const KArgs &a, hipStream_t s, bool &handled);
 hipError_t interleave_generic(const KArgs &a, hipStream_t s);
 hipError_t permute_fast(const KArgs &a, hipStream_t s, bool &handled);

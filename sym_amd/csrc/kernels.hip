@@ -23,6 +23,10 @@ hipError_t launch_box(int family, const KArgs &a, int32_t *status, hipStream_t s
   case kFamRaggedTranspose:
     e = transpose_ragged_fast(a, s, handled);
     return handled ? e : transpose_ragged_generic(a, s);
+  case kFamRows:
+  case kFamFlat:
+    e = rows_fast(a, s, handled);
+    return handled ? e : rows_generic(a, s);
   case kFamInterleave:
     e = interleave_fast(a, s, handled);
     return handled ? e : interleave_generic(a, s);

@@ -290,8 +290,30 @@ int row_mode(const HostStage &s, const Prepared &p, const Bound &b, int64_t len)
   return -1;
 }
 
+// Channel behaviour of V consecutive elements of a flat tensor from any
+// offset (DevStage::vec of k_flat): 0 per tensor, 2 at most two channels, 3 +1
+// per element and at most one wrap, -1 none of these.
+int flat_mode(const HostStage &s, const Prepared &p, const Bound &b, int64_t V) {
+  if (s.mode == kChanNone)
+    return 0;
+  if (s.mode != kChanDim)
+    return -1;
+  const int64_t rs = p.res_strides[static_cast<size_t>(s.dim)];
+  const int64_t re = b.result_extents[static_cast<size_t>(s.dim)];
+  if (re > s.len)
+    return -1;
+  if (rs == 1 && re >= V)
+    return 3;
+  return rs >= V ? 2 : -1;
+}
+
 bool transpose_family(int family) {
   return family == kFamTranspose || family == kFamRaggedTranspose;
+}
+
+// Families whose work items are vectors of the innermost axis.
+bool row_family(int family) {
+  return family == kFamStream || family == kFamRows || family == kFamFlat;
 }
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -486,11 +508,12 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
     return true;
   };
   // the same for kernels whose vectors start at any element of a row but
-  // never leave it: the channel is constant along a row, or the row's column
+  // never leave it (the channel is constant along a row, or the row's column),
+  // and for flat tensors
   const int64_t row_len = r > 0 ? pext[static_cast<size_t>(r - 1)] : 1;
-  auto row_channels_ok = [&] {
+  auto row_channels_ok = [&](bool flat = false) {
     for (uint32_t i = k; i < nst; ++i) {
-      const int m = row_mode(p.stages[i], p, b, row_len);
+      const int m = flat ? flat_mode(p.stages[i], p, b, V) : row_mode(p.stages[i], p, b, row_len);
       if (m < 0 || (p.stages[i].mode == kChanDim && !off32))
         return false;
       ch.st[i - k].vec = static_cast<uint8_t>(m);
@@ -566,6 +589,19 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
         family = kFamStream;
         a.vec = V;
         a.nlev = r <= 1 ? 1 : r <= 2 ? 2 : r <= 4 ? 4 : 8;
+      }
+    }
+    // rows, flat: the same axes where the vectors do not fit (at least one
+    // vector of valid elements; 32-bit columns)
+    if (family == kFamGeneric && a.ss[r - 1] == 1 && a.ds[r - 1] == 1 && a.vext[r - 1] >= V &&
+        row_len < kMaxLaunchWork - 64) {
+      if (r == 1 && !any_pad && row_channels_ok(true))
+        family = kFamFlat;
+      else if (row_channels_ok())
+        family = kFamRows;
+      if (family != kFamGeneric) {
+        a.vec = V;
+        a.nlev = r <= 2 ? 2 : r <= 4 ? 4 : 8;
       }
     }
     // transpose: dst-inner axis has a source stride, another axis is
@@ -652,7 +688,8 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
       ch.st[i - k].vec = 0;
   dp->family = family;
   a.chain_code = chain_code;
-  static const char *names[] = {"generic", "stream", "transpose", "interleave", "permute", "generic"};
+  static const char *names[] = {"generic", "stream", "transpose", "interleave", "permute",
+                                "generic", "generic", "generic"};
   dp->kernel = names[family];
 
   // ------------------------------------------------------- chunk axis
@@ -671,7 +708,7 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
       if (a.ss[ax] * a.vext[ax] == wire_elems && rest < a.ss[ax]) {
         dp->chunk_axis = ax;
         dp->chunk_stride = a.ss[ax];
-        if (family == kFamStream && ax == r - 1)
+        if (row_family(family) && ax == r - 1)
           dp->chunk_align = V;
         else if (transpose_family(family) && (ax == dp->qa || ax == dp->ca))
           dp->chunk_align = ax == dp->qa ? a.t_wq : a.t_wc;
@@ -707,8 +744,8 @@ int64_t box_work(const DeviceProgram &dp, const Box &b) {
   int64_t n = 1;
   for (int i = 0; i < r; ++i) {
     int64_t e = b.ext[i];
-    if (dp.family == kFamStream && i == r - 1)
-      e /= a.vec;
+    if (row_family(dp.family) && i == r - 1)
+      e = dp.family == kFamRows ? ceil_div(e, a.vec) : e / a.vec;
     else if (transpose_family(dp.family) && (i == dp.qa || i == dp.ca))
       e = ceil_div(e, i == dp.qa ? a.t_wq : a.t_wc);
     else if (dp.family == kFamInterleave && i == r - 2)
@@ -729,7 +766,7 @@ int64_t box_work(const DeviceProgram &dp, const Box &b) {
 // Coordinates a split of axis i must keep together (0: never split).
 int64_t split_align(const DeviceProgram &dp, int i) {
   const int r = dp.base.rank;
-  if (dp.family == kFamStream && i == r - 1)
+  if (row_family(dp.family) && i == r - 1)
     return dp.base.vec;
   if (transpose_family(dp.family) && (i == dp.qa || i == dp.ca))
     return i == dp.qa ? dp.base.t_wq : dp.base.t_wc;
@@ -929,6 +966,14 @@ bool permute_direct(KArgs &a, int64_t C, int64_t M, int64_t E) {
   return true;
 }
 
+// Valid source columns [lo, hi) of a box along the innermost axis.
+void valid_columns(const DeviceProgram &dp, const Box &b, int64_t &lo, int64_t &hi) {
+  const KArgs &a = dp.base;
+  const int i = a.rank - 1;
+  lo = std::max<int64_t>(0, b.lo[i] - a.lo[i]);
+  hi = std::min(a.vext[i], b.lo[i] + b.ext[i] - a.lo[i]);
+}
+
 // `family`: the program's own, or kFamRaggedTranspose for a box of a
 // transpose program whose last tiles are cut.
 KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
@@ -967,6 +1012,33 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
     for (int i = 0; i < r; ++i)
       a.lv[a.nlev - r + i] = axis_level(a, b, i, i == r - 1 ? a.vec : 1);
     break;
+  case kFamFlat: // a.work whole vectors and the tail
+    a.r_len = static_cast<uint32_t>(b.ext[0]);
+    work = b.ext[0] / a.vec;
+    break;
+  case kFamRows: {
+    for (int i = 0; i < r - 1; ++i)
+      a.lv[a.nlev - r + i] = axis_level(a, b, i, 1);
+    const int64_t n = ceil_div(b.ext[r - 1], a.vec);
+    Level &l = a.lv[a.nlev - 1]; // items of the row
+    l.div = make_div(n);
+    l.ss = l.ds = static_cast<uint32_t>(a.vec);
+    l.vlo = 0;
+    l.vcnt = static_cast<uint32_t>(n);
+    a.r_len = static_cast<uint32_t>(b.ext[r - 1]);
+    a.r_off = static_cast<int32_t>(b.lo[r - 1] - a.lo[r - 1]);
+    int64_t lo, hi;
+    valid_columns(dp, b, lo, hi);
+    a.r_lo = static_cast<int32_t>(lo);
+    a.r_hi = static_cast<int32_t>(hi);
+    // rows whose vectors are aligned stream their stores; others share a
+    // vector's line with the next row
+    bool aligned = (a.dbase * a.wout) % 16 == 0;
+    for (int i = 0; i < r - 1; ++i)
+      aligned = aligned && (a.ds[i] * a.wout) % 16 == 0;
+    a.r_nts = aligned ? 1 : 0;
+    break;
+  }
   case kFamTranspose:
     batch(dp.qa, dp.ca);
     {
@@ -1045,7 +1117,7 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
   }
   }
   a.work = family == kFamGeneric ? 0 : static_cast<uint32_t>(work);
-  a.work64 = work;
+  a.work64 = family == kFamFlat ? b.ext[0] : work; // a flat box may be a tail alone
   return a;
 }
 
@@ -1089,20 +1161,19 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
   }
   std::vector<KArgs> out;
   std::vector<Box> edges;
-  if (dp.family == kFamStream && a.rank == 1 && b.ext[0] % a.vec != 0) {
-    // the tail of a single contiguous axis (box starts are multiples of V)
-    const int64_t m = b.ext[0] / a.vec * a.vec;
-    Box e = b;
-    e.lo[0] = b.lo[0] + m;
-    e.ext[0] = b.ext[0] - m;
-    edges.push_back(e);
-    b.ext[0] = m;
-  }
   // A transpose box whose q or c extent is not a multiple of the tile runs
   // as one ragged launch; a small one keeps its whole tiles on the tile
   // kernel and runs the strips past them (the q strip over the whole c range,
   // the c strip beside the whole q tiles) as ragged launches.
   int family = dp.family;
+  if (family == kFamStream && a.rank == 1 && b.ext[0] % a.vec != 0)
+    family = kFamFlat; // the tail past the last vector in the same launch
+  if (family == kFamRows) { // a chunk of fewer valid columns than a vector
+    int64_t lo, hi;
+    valid_columns(dp, b, lo, hi);
+    if (hi - lo < a.vec)
+      return {edge_args(dp, b)};
+  }
   if (family == kFamTranspose && (b.ext[dp.qa] % a.t_wq || b.ext[dp.ca] % a.t_wc)) {
     if (box_elements(b, a.rank) >= kRaggedWholeElements) {
       family = kFamRaggedTranspose;
@@ -1135,8 +1206,7 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
       out.push_back(launch_args(dp, x, family));
   for (const Box &x : edges)
     if (box_elements(x, a.rank) > 0)
-      out.push_back(dp.family == kFamTranspose ? launch_args(dp, x, kFamRaggedTranspose)
-                                               : edge_args(dp, x));
+      out.push_back(launch_args(dp, x, kFamRaggedTranspose));
   return out;
 }
 
@@ -1309,6 +1379,58 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
           if (rowch && chan_of(a.chain.st[0], o) != a.t_choff + static_cast<uint32_t>(q0 + row))
             bad_launch(dp, "a row-indexed launch reads another parameter entry");
         }
+    }
+    break;
+  }
+  case kFamFlat: {
+    const int V = a.vec;
+    if (a.work64 >= kMaxLaunchWork || a.r_len != a.work64 || a.r_len / V != a.work)
+      bad_launch(dp, "work disagrees with the elements");
+    for (uint32_t i = 0; i <= a.work; ++i) { // the last one: the tail, element by element
+      const int n = i < a.work ? V : static_cast<int>(a.r_len % V);
+      if (n == 0)
+        break;
+      const int64_t s0 = a.sbase + int64_t{i} * V, d0 = a.dbase + int64_t{i} * V;
+      ck.src_run(s0, n, n == V);
+      ck.dst_run(d0, n, n == V);
+      for (int k = 0; k < a.chain.n; ++k) { // the entries k_flat takes
+        const DevStage &s = a.chain.st[k];
+        const uint32_t o = static_cast<uint32_t>(d0), c0 = chan_of(s, o), re = s.ch_re_div.d;
+        const uint32_t left = s.ch_rs_div.d - o % s.ch_rs_div.d;
+        for (int e = 0; e < n; ++e) {
+          uint32_t c = c0;
+          if (s.vec & 1)
+            c = c0 + e >= re ? c0 + e - re : c0 + e;
+          else if (s.vec != 0 && static_cast<uint32_t>(e) >= left)
+            c = c0 + 1 == re ? 0 : c0 + 1;
+          if (c != chan_of(s, d0 + e) || c >= s.len)
+            bad_launch(dp, "a flat launch reads another parameter entry");
+        }
+      }
+    }
+    break;
+  }
+  case kFamRows: {
+    if (a.work64 >= kMaxLaunchWork || a.work != a.work64)
+      bad_launch(dp, "work above 2^31");
+    const int V = a.vec;
+    const FastDiv &row_div = a.lv[a.nlev - 1].div;
+    if (a.r_hi - a.r_lo < V || ceil_div(a.r_len, V) != row_div.d)
+      bad_launch(dp, "columns disagree with the row's items");
+    for (uint32_t i = 0; i < a.work; ++i) { // the kernel's arithmetic
+      int64_t sof = a.sbase, dof = a.dbase;
+      bool pad = decompose_rt(a.nlev, a.lv, i, sof, dof);
+      const int32_t p = static_cast<int32_t>(i - fdiv(i, row_div) * row_div.d) * V;
+      const int32_t col = p + a.r_off, at = std::min(std::max(col, a.r_lo), a.r_hi - V);
+      pad |= col >= a.r_hi || col + V <= a.r_lo;
+      const int n = std::min<int>(V, static_cast<int>(a.r_len) - p);
+      ck.dst_run(dof, n, a.r_nts && n == V);
+      if (!pad) {
+        if (std::abs(at - col) >= V)
+          bad_launch(dp, "a vector moves by its whole width");
+        ck.src_run(sof + (at - col), V, false);
+        ck.channels(dof, n);
+      }
     }
     break;
   }
@@ -1494,7 +1616,8 @@ int64_t launch_all(const DeviceProgram &dp, std::vector<KArgs> launches, const v
                        reinterpret_cast<uintptr_t>(dst) % 16 == 0;
   int64_t n = 0;
   for (KArgs &a : launches) {
-    if (!aligned && a.family != kFamGeneric && a.family != kFamRaggedTranspose) {
+    if (!aligned && a.family != kFamGeneric && a.family != kFamRaggedTranspose &&
+        a.family != kFamRows) {
       a.family = kFamGeneric;
       int64_t e = 1;
       for (int i = 0; i < a.rank; ++i)

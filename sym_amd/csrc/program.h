@@ -83,7 +83,8 @@ struct DevStage {
   uint8_t op;
   uint8_t mode;
   uint8_t zp_per_ch; // zero point has one entry per channel
-  uint8_t vec;       // vector kernels: 0 channel constant across a vector, 1 +1 per element
+  uint8_t vec;       // vector kernels: 0 channel constant across a vector, 1 +1 per element;
+                     // flat: 2 at most two channels in a vector, 3 +1 per element, wrapping
   uint32_t scale_off; // float param index (dequant scale / quant reciprocal)
   uint32_t zp_off;    // int param index
   uint32_t len;       // parameter entries
@@ -109,6 +110,8 @@ enum Family : int32_t {
   kFamInterleave = 3, // planar -> interleaved with a small padded inner axis
   kFamPermute = 4,    // swap of two axes above a contiguous inner block, through LDS
   kFamRaggedTranspose = 5, // batched 2-D transpose of any extents and row alignments
+  kFamRows = 6, // innermost axis contiguous on both sides, rows of any length, alignment and pads
+  kFamFlat = 7, // one contiguous axis whose channels or length fit no whole vectors
 };
 
 // Tiles of the ragged transpose: 64 q by 64 c, or large ones 128 c wide
@@ -227,6 +230,12 @@ struct KArgs {
   // ragged transpose: extents of q and c in the box (the last tile along
   // either may be cut)
   uint32_t t_qn, t_cn;
+  // rows: destination columns in the box (flat: elements), the source column
+  // of the first one (negative in a leading pad), the valid source columns
+  // [r_lo, r_hi) of the box, streaming stores
+  uint32_t r_len;
+  int32_t r_off, r_lo, r_hi;
+  uint32_t r_nts;
   // ---- generic kernel and host bookkeeping (coalesced destination axes)
   int32_t rank;
   int32_t win, wout; // element bytes of the wire and of the result

@@ -39,9 +39,10 @@ def _chains(shape, axis, rng):
 def _source(shape, dtype, rng):
     if dtype == "int8":
         return rng.integers(-128, 128, shape, dtype=np.int8)
-    x = rng.standard_normal(shape) * 3
-    x.reshape(-1)[:: 97] = np.resize([np.nan, np.inf, -np.inf, -0.0, 1e30, 1e-30], x.reshape(-1)[::97].size)
-    return x.astype(dtype)
+    x = (rng.standard_normal(shape) * 3).astype(dtype)
+    x.reshape(-1)[:: 97] = np.resize(np.array([np.nan, np.inf, -np.inf, -0.0, 6e4, 1e-7], dtype),
+                                     x.reshape(-1)[::97].size)
+    return x
 
 
 # (rows, cols) [batch] around the tile widths: one row of a vector less or
@@ -63,8 +64,53 @@ def transpose_cases(case):
                 _source(shape, dtype, rng)
 
 
+# (shape, pads as (axis, lo, hi), outer permutation): pads that begin and end
+# inside a vector, rows of one vector and of one element more, padded outer
+# axes, odd rows under swapped outer axes
+ROWS = [((5, 16), ((1, 0, 1),), None), ((7, 17), ((1, 3, 0),), None), ((33, 1003), ((1, 0, 21),), None),
+        ((9, 130), ((1, 5, 7),), None), ((6, 65), ((0, 1, 2), (1, 1, 0)), None), ((1, 300), ((1, 2, 3),), None),
+        ((3, 4, 5, 35), (), (0, 2, 1, 3)), ((3, 5, 67), (), (1, 0, 2)), ((2, 3, 5, 21), ((3, 1, 1),), None)]
+
+
+def rows_cases(case):
+    shape, pads, perm = case
+    rng = np.random.default_rng(sum(shape))
+    for axis in [None] + list(range(len(shape))):
+        for dtype, ops in _chains(shape, axis, rng):
+            params = any(isinstance(o, (EN.Dequantize, EN.Quantize)) for o in ops)
+            if axis is not None and not params:
+                continue
+            layout = [EN.Pad(a, lo, hi, 3 if dtype == "int8" else 1.5) for a, lo, hi in pads]
+            layout += [EN.Transpose(perm)] if perm else []
+            # a fill cannot cross a per-channel stage: the pad follows it
+            ops = layout + ops if axis is None else ops + layout
+            try:
+                plan = EN.encode(list(shape), dtype, ops)
+            except EN.EncodeError:
+                continue
+            yield "%s %s axis %s %s" % (dtype, shape, axis, [type(o).__name__ for o in ops]), plan.blob, \
+                _source(shape, dtype, rng)
+
+
+# flat tensors: channels of rows shorter and longer than a vector that start
+# inside one, one channel per column with the wrap inside a vector, tails of
+# every length class
+FLAT = [(3, 17), (37, 16), (50, 21), (129, 67), (11, 4099), (1, 1027), (2053, 33)]
+
+
+def flat_cases(shape):
+    rng = np.random.default_rng(shape[0] * 31 + shape[1])
+    for axis in (None, 0, 1):
+        for dtype, ops in _chains(shape, axis, rng):
+            plan = EN.encode(list(shape), dtype, ops)
+            yield "%s %s axis %s %s" % (dtype, shape, axis, [type(o).__name__ for o in ops]), plan.blob, \
+                _source(shape, dtype, rng)
+
+
 GROUPS = [("transpose", c, transpose_cases) for c in TRANSPOSES]
-IDS = ["%s %s" % (k, "x".join(str(v) for v in c if v is not None)) for k, c, _ in GROUPS]
+GROUPS += [("rows", c, rows_cases) for c in ROWS]
+GROUPS += [("flat", c, flat_cases) for c in FLAT]
+IDS = ["%s %s" % (k, c) for k, c, _ in GROUPS]
 
 
 @pytest.mark.parametrize("group", GROUPS, ids=IDS)
