@@ -14,17 +14,6 @@
 namespace relx {
 namespace {
 
-// v moved down (towards byte 0) by n < 16 bytes, zeros behind it.
-__device__ __forceinline__ vec4 down_bytes(vec4 v, uint32_t n) {
-  if (n & 8)
-    v = vec4{v.z, v.w, 0u, 0u};
-  if (n & 4)
-    v = vec4{v.y, v.z, v.w, 0u};
-  const uint32_t b = (n & 3) * 8;
-  return vec4{__builtin_amdgcn_alignbit(v.y, v.x, b), __builtin_amdgcn_alignbit(v.z, v.y, b),
-              __builtin_amdgcn_alignbit(v.w, v.z, b), v.w >> b};
-}
-
 // v moved up by n < 16 bytes, zeros before it.
 __device__ __forceinline__ vec4 up_bytes(vec4 v, uint32_t n) {
   if (n & 8)

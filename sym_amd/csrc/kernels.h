@@ -626,6 +626,17 @@ __device__ __forceinline__ void stu_cut(uint8_t *p, vec4 v, uint32_t n) {
     *p = static_cast<uint8_t>(v.x);
 }
 
+// v moved down (towards byte 0) by n < 16 bytes, zeros behind it.
+__device__ __forceinline__ vec4 down_bytes(vec4 v, uint32_t n) {
+  if (n & 8)
+    v = vec4{v.z, v.w, 0u, 0u};
+  if (n & 4)
+    v = vec4{v.y, v.z, v.w, 0u};
+  const uint32_t b = (n & 3) * 8;
+  return vec4{__builtin_amdgcn_alignbit(v.y, v.x, b), __builtin_amdgcn_alignbit(v.z, v.y, b),
+              __builtin_amdgcn_alignbit(v.w, v.z, b), v.w >> b};
+}
+
 // ---------------------------------------------------------------- stream
 
 // Stream work items hold V = 16/max(win, wout) elements: the wider side
@@ -1616,6 +1627,8 @@ hipError_t rows_fast(const KArgs &a, hipStream_t s, bool &handled);
 hipError_t rows_generic(const KArgs &a, hipStream_t s);
 hipError_t interleave_fast(const KArgs &a, hipStream_t s, bool &handled);
 hipError_t interleave_generic(const KArgs &a, hipStream_t s);
+hipError_t interleave_ragged_fast(const KArgs &a, hipStream_t s, bool &handled);
+hipError_t interleave_ragged_generic(const KArgs &a, hipStream_t s);
 hipError_t permute_fast(const KArgs &a, hipStream_t s, bool &handled);
 hipError_t permute_generic(const KArgs &a, hipStream_t s);
 

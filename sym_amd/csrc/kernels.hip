@@ -27,6 +27,9 @@ hipError_t launch_box(int family, const KArgs &a, int32_t *status, hipStream_t s
   case kFamFlat:
     e = rows_fast(a, s, handled);
     return handled ? e : rows_generic(a, s);
+  case kFamRaggedInterleave:
+    e = interleave_ragged_fast(a, s, handled);
+    return handled ? e : interleave_ragged_generic(a, s);
   case kFamInterleave:
     e = interleave_fast(a, s, handled);
     return handled ? e : interleave_generic(a, s);

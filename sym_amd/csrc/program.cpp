@@ -307,6 +307,10 @@ int flat_mode(const HostStage &s, const Prepared &p, const Bound &b, int64_t V) 
   return rs >= V ? 2 : -1;
 }
 
+bool interleave_family(int family) {
+  return family == kFamInterleave || family == kFamRaggedInterleave;
+}
+
 bool transpose_family(int family) {
   return family == kFamTranspose || family == kFamRaggedTranspose;
 }
@@ -668,14 +672,16 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
       const int G = interleave_pixels(win, wout, static_cast<int>(cp));
       const int64_t bo = G * cp * wout;
       bool pa_pad = lo[static_cast<size_t>(r - 2)] != 0 || pext[static_cast<size_t>(r - 2)] != a.vext[r - 2];
-      bool ok = (cp == 2 || cp == 4 || cp == 8) && !pa_pad && a.vext[r - 2] % G == 0 &&
-                a.ss[r - 1] % G == 0 && (bo == 4 || bo == 8 || bo % 16 == 0);
-      for (int i = 0; i < r - 2; ++i)
-        ok = ok && a.ss[i] % G == 0;
+      bool ok = (cp == 2 || cp == 4 || cp == 8) && !pa_pad && a.vext[r - 2] >= G &&
+                (bo == 4 || bo == 8 || bo % 16 == 0);
       for (uint32_t i = k; i < nst; ++i)
         ok = ok && p.stages[i].mode == kChanNone;
+      // whole groups at aligned planes, or any
+      bool whole = a.vext[r - 2] % G == 0 && a.ss[r - 1] % G == 0;
+      for (int i = 0; i < r - 2; ++i)
+        whole = whole && a.ss[i] % G == 0;
       if (ok) {
-        family = kFamInterleave;
+        family = whole ? kFamInterleave : kFamRaggedInterleave;
         a.vec = G;
         a.cpad = static_cast<int32_t>(cp);
       }
@@ -689,7 +695,7 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
   dp->family = family;
   a.chain_code = chain_code;
   static const char *names[] = {"generic", "stream", "transpose", "interleave", "permute",
-                                "generic", "generic", "generic"};
+                                "generic", "generic", "generic", "generic"};
   dp->kernel = names[family];
 
   // ------------------------------------------------------- chunk axis
@@ -712,11 +718,11 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
           dp->chunk_align = V;
         else if (transpose_family(family) && (ax == dp->qa || ax == dp->ca))
           dp->chunk_align = ax == dp->qa ? a.t_wq : a.t_wc;
-        else if (family == kFamInterleave && ax == r - 2)
+        else if (interleave_family(family) && ax == r - 2)
           dp->chunk_align = a.vec;
         // an interleave launch writes every channel of its pixels, so its
         // boxes never split the channel axis
-        if (family == kFamInterleave && ax == r - 1)
+        if (interleave_family(family) && ax == r - 1)
           dp->chunk_axis = -1;
         // a permute block takes T rows of m and all of c and e
         if (family == kFamPermute) {
@@ -748,9 +754,9 @@ int64_t box_work(const DeviceProgram &dp, const Box &b) {
       e = dp.family == kFamRows ? ceil_div(e, a.vec) : e / a.vec;
     else if (transpose_family(dp.family) && (i == dp.qa || i == dp.ca))
       e = ceil_div(e, i == dp.qa ? a.t_wq : a.t_wc);
-    else if (dp.family == kFamInterleave && i == r - 2)
-      e /= a.vec;
-    else if (dp.family == kFamInterleave && i == r - 1)
+    else if (interleave_family(dp.family) && i == r - 2)
+      e = ceil_div(e, a.vec);
+    else if (interleave_family(dp.family) && i == r - 1)
       e = 1;
     else if (dp.family == kFamPermute && i == r - 2)
       e /= a.p_t;
@@ -770,9 +776,9 @@ int64_t split_align(const DeviceProgram &dp, int i) {
     return dp.base.vec;
   if (transpose_family(dp.family) && (i == dp.qa || i == dp.ca))
     return i == dp.qa ? dp.base.t_wq : dp.base.t_wc;
-  if (dp.family == kFamInterleave && i == r - 2)
+  if (interleave_family(dp.family) && i == r - 2)
     return dp.base.vec;
-  if (dp.family == kFamInterleave && i == r - 1)
+  if (interleave_family(dp.family) && i == r - 1)
     return 0;
   if (dp.family == kFamPermute && i == r - 2)
     return dp.base.p_t;
@@ -787,7 +793,7 @@ bool level_axis(const DeviceProgram &dp, int i) {
   const int r = dp.base.rank;
   if (transpose_family(dp.family))
     return i != dp.qa && i != dp.ca;
-  if (dp.family == kFamInterleave)
+  if (interleave_family(dp.family))
     return i < r - 2;
   if (dp.family == kFamPermute)
     return i < r - 3;
@@ -989,7 +995,7 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
   a.sbase = 0;
   a.dbase = 0;
   for (int i = 0; i < r; ++i) {
-    if (dp.family == kFamInterleave && i == r - 1)
+    if (interleave_family(dp.family) && i == r - 1)
       continue;
     a.sbase += (b.lo[i] - a.lo[i]) * a.ss[i];
     a.dbase += b.lo[i] * a.ds[i];
@@ -1106,8 +1112,10 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
     break;
   }
   case kFamInterleave:
+  case kFamRaggedInterleave:
     batch(r - 2, r - 1);
-    a.i_ng = make_div(b.ext[r - 2] / a.vec);
+    a.r_len = static_cast<uint32_t>(b.ext[r - 2]);
+    a.i_ng = make_div(ceil_div(b.ext[r - 2], a.vec));
     a.i_ssc = a.ss[r - 1];
     a.i_loc = static_cast<int32_t>(a.lo[r - 1]);
     a.i_vc = static_cast<int32_t>(a.vext[r - 1]);
@@ -1174,6 +1182,9 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
     if (hi - lo < a.vec)
       return {edge_args(dp, b)};
   }
+  // a chunk of fewer pixels than a group
+  if (family == kFamRaggedInterleave && b.ext[a.rank - 2] < a.vec)
+    return {edge_args(dp, b)};
   if (family == kFamTranspose && (b.ext[dp.qa] % a.t_wq || b.ext[dp.ca] % a.t_wc)) {
     if (box_elements(b, a.rank) >= kRaggedWholeElements) {
       family = kFamRaggedTranspose;
@@ -1480,14 +1491,18 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
     }
     break;
   }
+  case kFamRaggedInterleave:
   case kFamInterleave: {
     if (a.work64 >= kMaxLaunchWork || a.work != a.work64)
       bad_launch(dp, "work above 2^31");
+    const bool rag = dp.family == kFamRaggedInterleave;
     const int G = a.vec, CP = a.cpad;
     for (int k = 0; k < a.chain.n; ++k)
       if (a.chain.st[k].mode != kChanNone)
         bad_launch(dp, "per-channel stage in an interleave program");
-    if ((a.i_ssc * win) % (G * win) != 0)
+    if (a.r_len < static_cast<uint32_t>(G) || a.i_ng.d != ceil_div(a.r_len, G))
+      bad_launch(dp, "pixel groups disagree with the box");
+    if (!rag && (a.i_ssc * win) % (G * win) != 0)
       bad_launch(dp, "plane stride breaks the alignment of plane loads");
     if (G != interleave_pixels(win, wout, CP))
       bad_launch(dp, "pixels per item disagree with the kernel");
@@ -1496,12 +1511,14 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
       const uint32_t g = i - rest * a.i_ng.d;
       int64_t sbase = a.sbase, dbase = a.dbase;
       const bool pad = decompose_rt(kBatchLevels, a.lv, rest, sbase, dbase);
-      const int64_t p0 = int64_t{g} * G;
-      ck.dst_run(dbase + p0 * CP, int64_t{G} * CP, true);
+      const int64_t p0 = int64_t{g} * G, back = std::max<int64_t>(0, p0 + G - a.r_len);
+      if (back && !rag)
+        bad_launch(dp, "a cut pixel group");
+      ck.dst_run(dbase + p0 * CP, (G - back) * CP, !rag);
       for (int c = 0; c < CP; ++c) {
         const int32_t vc = c - a.i_loc;
         if (!pad && static_cast<uint32_t>(vc) < static_cast<uint32_t>(a.i_vc))
-          ck.src_run(sbase + vc * a.i_ssc + p0, G, true);
+          ck.src_run(sbase + vc * a.i_ssc + p0 - back, G, !rag);
       }
     }
     break;
@@ -1617,7 +1634,7 @@ int64_t launch_all(const DeviceProgram &dp, std::vector<KArgs> launches, const v
   int64_t n = 0;
   for (KArgs &a : launches) {
     if (!aligned && a.family != kFamGeneric && a.family != kFamRaggedTranspose &&
-        a.family != kFamRows) {
+        a.family != kFamRows && a.family != kFamRaggedInterleave) {
       a.family = kFamGeneric;
       int64_t e = 1;
       for (int i = 0; i < a.rank; ++i)

@@ -111,6 +111,7 @@ enum Family : int32_t {
   kFamPermute = 4,    // swap of two axes above a contiguous inner block, through LDS
   kFamRaggedTranspose = 5, // batched 2-D transpose of any extents and row alignments
   kFamRows = 6, // innermost axis contiguous on both sides, rows of any length, alignment and pads
+  kFamRaggedInterleave = 8, // planar -> interleaved, any pixel count and plane alignment
   kFamFlat = 7, // one contiguous axis whose channels or length fit no whole vectors
 };
 
@@ -230,7 +231,8 @@ struct KArgs {
   // ragged transpose: extents of q and c in the box (the last tile along
   // either may be cut)
   uint32_t t_qn, t_cn;
-  // rows: destination columns in the box (flat: elements), the source column
+  // rows: destination columns in the box (flat: elements, ragged interleave:
+  // pixels), the source column
   // of the first one (negative in a leading pad), the valid source columns
   // [r_lo, r_hi) of the box, streaming stores
   uint32_t r_len;

@@ -107,7 +107,26 @@ def flat_cases(shape):
                 _source(shape, dtype, rng)
 
 
+# ([batch..., C, H, W], leading and trailing channel pad) to two, four or
+# eight interleaved channels: pixel counts that cut the last pixel group at
+# every place, one group, planes of one batch entry after another
+IMAGES = [((2, 3, 3, 5), (0, 1)), ((3, 1, 17, 19), (1, 0)), ((1, 3, 4, 4), (1, 0)), ((2, 5, 9, 11), (1, 2)),
+          ((5, 4, 25, 41), (0, 0)), ((2, 2, 3, 7, 13), (0, 1)), ((4, 7, 3, 7), (0, 1)), ((1, 2, 1, 1027), (0, 0))]
+
+
+def image_cases(case):
+    shape, (lo, hi) = case
+    rng = np.random.default_rng(sum(shape))
+    n = len(shape)
+    perm = tuple(range(n - 3)) + (n - 2, n - 1, n - 3)
+    for dtype, ops in _chains(shape, None, rng):
+        layout = ([EN.Pad(n - 3, lo, hi, 3 if dtype == "int8" else 1.5)] if lo + hi else []) + [EN.Transpose(perm)]
+        plan = EN.encode(list(shape), dtype, layout + ops)
+        yield "%s %s %s" % (dtype, shape, [type(o).__name__ for o in ops]), plan.blob, _source(shape, dtype, rng)
+
+
 GROUPS = [("transpose", c, transpose_cases) for c in TRANSPOSES]
+GROUPS += [("image", c, image_cases) for c in IMAGES]
 GROUPS += [("rows", c, rows_cases) for c in ROWS]
 GROUPS += [("flat", c, flat_cases) for c in FLAT]
 IDS = ["%s %s" % (k, c) for k, c, _ in GROUPS]
