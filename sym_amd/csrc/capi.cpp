@@ -371,7 +371,7 @@ int relx_bound_query(const relx_bound *bound, relx_bound_info *out) {
       const std::vector<relx::KArgs> ls = relx::axis_launches(dp, -1, 0, 0);
       out->permute_direct = ls.empty() ? 0 : 1;
       for (const relx::KArgs &a : ls)
-        if (!a.p_direct)
+        if (a.p_direct != relx::kPermuteShift)
           out->permute_direct = 0;
     }
     if (!b.typed)

@@ -1257,9 +1257,11 @@ __device__ __forceinline__ void chain_vec_direct(uint32_t (&v)[V], const VecPara
 }
 
 // The permute of a direct launch: the same blocks, tile and store order from
-// PermArgs, with shifts and masks for the divisions inside a block, the batch
-// entry's offset as one multiply, and a vector's parameters by its channel.
-template <int WIN, int WOUT, int CH>
+// PermArgs, the batch entry's offset as one multiply, and a vector's
+// parameters by its channel. SHIFT: G*E, E and a run are powers of two (shifts
+// and masks for the divisions inside a block) and T divides the box's m;
+// otherwise the divisions are FastDivs and the last m-tile may be cut.
+template <int WIN, int WOUT, int CH, bool SHIFT>
 __device__ __forceinline__ void permute_direct_body(const PermArgs &a) {
   static_assert(CH != kChainGeneric, "direct launches run compile-time chains");
   extern __shared__ __align__(16) uint8_t lds[];
@@ -1275,6 +1277,9 @@ __device__ __forceinline__ void permute_direct_body(const PermArgs &a) {
                "s"(a.bss), "s"(a.bds), "s"(a.nout), "s"(a.cmask), "s"(a.scale_off));
   if constexpr (CH == kChainDeqF16 || CH == kChainDeq)
     asm volatile("" ::"s"(a.pi), "s"(a.zp_off), "s"(a.zp_per_ch));
+  if constexpr (!SHIFT)
+    asm volatile("" ::"s"(a.ge_d), "s"(a.ge_m), "s"(a.e_d), "s"(a.e_m), "s"(a.run_d), "s"(a.run_m),
+                 "s"(a.m));
   const uint32_t t = blockIdx.x;
   if (t >= a.work)
     return;
@@ -1282,20 +1287,26 @@ __device__ __forceinline__ void permute_direct_body(const PermArgs &a) {
   const uint32_t t2 = t - cg * a.cgt_d;
   const uint32_t b = fdiv(t2, FastDiv{a.tiles_d, a.tiles_m, a.tiles_s, 0});
   const uint32_t m0 = (t2 - b * a.tiles_d) * a.t, c0 = cg * a.g;
-  const uint32_t GE = 1u << a.ge_s, E = 1u << a.e_s;
+  const uint32_t GE = SHIFT ? 1u << a.ge_s : a.ge_d, E = SHIFT ? 1u << a.e_s : a.e_d;
+  auto div_ge = [&](uint32_t x) { return SHIFT ? x >> a.ge_s : fdiv(x, FastDiv{a.ge_d, a.ge_m, a.ge_s, 0}); };
+  auto div_e = [&](uint32_t x) { return SHIFT ? x >> a.e_s : fdiv(x, FastDiv{a.e_d, a.e_m, a.e_s, 0}); };
+  auto div_run = [&](uint32_t x) {
+    return SHIFT ? x >> a.run_s : fdiv(x, FastDiv{a.run_d, a.run_m, a.run_s, 0});
+  };
+  const uint32_t rows = SHIFT ? a.t : min(a.t, a.m - m0); // m of this block
   const vec4 *src = reinterpret_cast<const vec4 *>(
       a.src + (a.sbase + static_cast<int64_t>(b) * a.bss + static_cast<int64_t>(m0) * a.ce +
                static_cast<int64_t>(c0) * E) * WIN);
   const uint32_t gap = (a.ce - GE) / VI; // vectors between two row parts
-  const uint32_t nvec = (a.t << a.ge_s) / VI;
+  const uint32_t nvec = SHIFT ? (a.t << a.ge_s) / VI : rows * GE / VI;
   for (uint32_t v0 = threadIdx.x; v0 < nvec; v0 += kBlock * U) {
     uint32_t tt[U], rem[U];
     vec4 in[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t v = v0 + u * kBlock < nvec ? v0 + u * kBlock : v0;
-      tt[u] = (v * VI) >> a.ge_s;
-      rem[u] = (v * VI) & (GE - 1);
+      tt[u] = div_ge(v * VI);
+      rem[u] = v * VI - tt[u] * GE;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -1307,7 +1318,7 @@ __device__ __forceinline__ void permute_direct_body(const PermArgs &a) {
     VecParams par[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint32_t cl = rem[u] >> a.e_s, e = rem[u] & (E - 1);
+      const uint32_t cl = div_e(rem[u]), e = rem[u] - cl * E;
       lds_off[u] = ((cl * a.t + tt[u]) * E + e) * WOUT;
       par[u] = direct_params<CH>(a, (c0 + cl) & a.cmask);
     }
@@ -1336,12 +1347,14 @@ __device__ __forceinline__ void permute_direct_body(const PermArgs &a) {
   __syncthreads();
   uint8_t *dst = a.dst + (a.dbase + static_cast<int64_t>(b) * a.bds + static_cast<int64_t>(c0) * a.dsc +
                           static_cast<int64_t>(m0) * E) * WOUT;
-  const uint32_t rmask = (1u << a.run_s) - 1;
+  const uint32_t run = SHIFT ? 1u << a.run_s : a.run_d;
+  const uint32_t live = rows * E * WOUT / 16; // vectors of a run that hold this block's m
   for (uint32_t w = threadIdx.x; w < a.nout; w += kBlock) {
+    const uint32_t cl = div_run(w), j = w - cl * run;
+    if (!SHIFT && j >= live)
+      continue;
     const vec4 val = reinterpret_cast<const vec4 *>(lds)[w];
-    st16<NTS>(reinterpret_cast<vec4 *>(dst + static_cast<int64_t>(w >> a.run_s) * a.dsc * WOUT) +
-                  (w & rmask),
-              val);
+    st16<NTS>(reinterpret_cast<vec4 *>(dst + static_cast<int64_t>(cl) * a.dsc * WOUT) + j, val);
   }
 }
 
@@ -1363,13 +1376,24 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 
 template <int WIN, int WOUT, int CH>
 __global__ __launch_bounds__(kBlock) void k_permute_direct(PermArgs a) {
-  permute_direct_body<WIN, WOUT, CH>(a);
+  permute_direct_body<WIN, WOUT, CH, true>(a);
+}
+
+template <int WIN, int WOUT, int CH>
+__global__ __launch_bounds__(kBlock) void k_permute_div(PermArgs a) {
+  permute_direct_body<WIN, WOUT, CH, false>(a);
 }
 
 template <int WIN, int WOUT, int CH>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_permute_direct8(
     PermArgs a) {
-  permute_direct_body<WIN, WOUT, CH>(a);
+  permute_direct_body<WIN, WOUT, CH, true>(a);
+}
+
+template <int WIN, int WOUT, int CH>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_permute_div8(
+    PermArgs a) {
+  permute_direct_body<WIN, WOUT, CH, false>(a);
 }
 
 // ------------------------------------------------------------ launch
@@ -1471,8 +1495,8 @@ hipError_t interleave_cp(const KArgs &a, hipStream_t s) {
   }
 }
 
-// A direct launch's PermArgs (KArgs::p_direct; the host has proven the shifts,
-// the channel entries and a single batch level).
+// A direct launch's PermArgs (KArgs::p_direct; the host has proven the shifts
+// of a shift launch, the channel entries and a single batch level).
 inline PermArgs permute_direct_args(const KArgs &a) {
   PermArgs p{};
   p.src = a.src;
@@ -1494,6 +1518,13 @@ inline PermArgs permute_direct_args(const KArgs &a) {
   p.ge_s = a.p_ge.s;
   p.e_s = a.p_e.s;
   p.run_s = a.p_run.s;
+  p.ge_d = a.p_ge.d;
+  p.ge_m = a.p_ge.m;
+  p.e_d = a.p_e.d;
+  p.e_m = a.p_e.m;
+  p.run_d = a.p_run.d;
+  p.run_m = a.p_run.m;
+  p.m = a.p_m;
   p.ce = a.p_ce.d;
   p.bss = a.lv[kBatchLevels - 1].ss;
   p.bds = a.lv[kBatchLevels - 1].ds;
@@ -1514,10 +1545,18 @@ hipError_t permute_launch(const KArgs &a, hipStream_t s) {
   if constexpr (CH != kChainGeneric) {
     if (a.p_direct) {
       const PermArgs p = permute_direct_args(a);
-      if constexpr (permute_eight_waves(WIN, CH))
-        hipLaunchKernelGGL((k_permute_direct8<WIN, WOUT, CH>), grid, block, a.p_lds, s, p);
-      else
-        hipLaunchKernelGGL((k_permute_direct<WIN, WOUT, CH>), grid, block, a.p_lds, s, p);
+      const bool shift = a.p_direct == kPermuteShift;
+      if constexpr (permute_eight_waves(WIN, CH)) {
+        if (shift)
+          hipLaunchKernelGGL((k_permute_direct8<WIN, WOUT, CH>), grid, block, a.p_lds, s, p);
+        else
+          hipLaunchKernelGGL((k_permute_div8<WIN, WOUT, CH>), grid, block, a.p_lds, s, p);
+      } else {
+        if (shift)
+          hipLaunchKernelGGL((k_permute_direct<WIN, WOUT, CH>), grid, block, a.p_lds, s, p);
+        else
+          hipLaunchKernelGGL((k_permute_div<WIN, WOUT, CH>), grid, block, a.p_lds, s, p);
+      }
       return hipGetLastError();
     }
   }

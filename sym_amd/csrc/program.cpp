@@ -365,6 +365,49 @@ constexpr int64_t kRaggedWholeElements = int64_t{1} << 14;
 // Shortest q and c extents that take the ragged transpose's tiles.
 constexpr int64_t kRaggedMinExtent = 16;
 
+// A chain that a direct permute of planes of `rs` elements and C channels can
+// run: a compile-time one whose parameter stage is per tensor or along c.
+bool direct_chain(const Bound &b, const Prepared &p, uint32_t k, int chain_code, int64_t rs, int64_t C) {
+  if (chain_code == kChainGeneric)
+    return false;
+  const int at = chain_param_stage(chain_code);
+  if (at < 0)
+    return true;
+  const HostStage &s = p.stages[k + static_cast<uint32_t>(at)];
+  if (s.mode == kChanNone)
+    return true;
+  return s.mode == kChanDim && p.res_strides[static_cast<size_t>(s.dim)] == rs &&
+         b.result_extents[static_cast<size_t>(s.dim)] == C;
+}
+
+// Channels G (a divisor of C, at most RELX_PERMUTE_GROUP_BYTES of a source
+// row) and rows T of a direct permute's block: the pair whose blocks keep the
+// most of their 256 lanes busy, the cut last m-tile counted, over at most
+// three vectors per lane; among equals the longer row part. f16 -> int8 on the
+// MI355X, general kernel and power-of-two rule -> here: [61,184,40,128] 57.3 ->
+// 30.0 us (10 channels of one row, 160 vectors -> 8 of two, 256), [50,150,32,96]
+// 23.1 -> 14.4 us (192 -> 768), [33,999,8,128] 23.5 -> 17.7 us (odd m: 128 ->
+// 768).
+void permute_block(int64_t C, int64_t M, int64_t E, int win, int wout, int64_t &G, int64_t &T) {
+  double best = 0.0;
+  for (int64_t g = C; g >= 1; --g) {
+    if (C % g || (g * E * win > RELX_PERMUTE_GROUP_BYTES && g > 1))
+      continue;
+    for (int64_t t = 1; t <= std::min<int64_t>(8, M); ++t) {
+      const int64_t n = t * g * E * win / 16;
+      if (t * g * E * wout > 32768 || (n > 3 * 256 && t > 1))
+        continue;
+      const double use = static_cast<double>(n) / static_cast<double>(ceil_div(n, 256) * 256) *
+                         static_cast<double>(M) / static_cast<double>(ceil_div(M, t) * t);
+      if (use > best + 1e-9) {
+        best = use;
+        G = g;
+        T = t;
+      }
+    }
+  }
+}
+
 } // namespace
 
 std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, uint32_t k) {
@@ -572,6 +615,11 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
         T *= 2;
       ok = T * G * E * wout <= 32768;
     }
+    // blocks that leave lanes idle (their vectors are not a multiple of the
+    // 256 lanes) take another G and T where the launches run the direct
+    // kernel, whose last m-tile may be cut
+    if (ok && (T * G * E / VI) % 256 != 0 && c <= 1 && direct_chain(b, p, k, chain_code, M * E, C))
+      permute_block(C, M, E, win, wout, G, T);
     if (ok && channels_ok(VI)) {
       family = kFamPermute;
       a.vec = VI;
@@ -759,7 +807,7 @@ int64_t box_work(const DeviceProgram &dp, const Box &b) {
     else if (interleave_family(dp.family) && i == r - 1)
       e = 1;
     else if (dp.family == kFamPermute && i == r - 2)
-      e /= a.p_t;
+      e = ceil_div(e, a.p_t); // cut only where the direct kernel runs
     else if (dp.family == kFamPermute && i == r - 3)
       e /= a.p_g;
     else if (dp.family == kFamPermute && i > r - 3)
@@ -936,40 +984,44 @@ bool zero_points_zero(const DeviceProgram &dp, const DevStage &s, int64_t c0, in
   return true;
 }
 
-// A permute launch runs the direct body when its divisions are shifts (G*E,
-// E and the 16-byte vectors of a run are powers of two, so make_div gives
-// m = 1 and s = log2 d), its batch entries lie along one level (the outer
-// levels are unit levels) and the parameter stage, if any, takes a vector's
-// entry from the block's own c coordinate. For a stage per channel along c
+// A permute launch runs the direct body when its batch entries lie along one
+// level (the outer levels are unit levels) and the parameter stage, if any,
+// takes a vector's entry from the block's own c coordinate: with shifts when
+// G*E, E and the 16-byte vectors of a run are powers of two (make_div then
+// gives m = 1 and s = log2 d) and T divides the box's m, else with divisions
+// and a last m-tile that may be cut. For a stage per channel along c
 // (rs = M*E, re = C) at result offset o = D + c*M*E + m*E + e, with m < M,
 // e < E and D the offset of the block's batch entry, (o / (M*E)) mod C = c
 // exactly when D is a multiple of C*M*E: every batch level's destination
 // stride is, and the launch origin is one plus an offset inside a plane
 // (below M*E; a launch may start at any m). A per-tensor stage takes entry 0.
-bool permute_direct(KArgs &a, int64_t C, int64_t M, int64_t E) {
+int permute_direct(KArgs &a, int64_t C, int64_t M, int64_t E) {
   a.p_cmask = 0;
-  if (a.chain_code == kChainGeneric || !pow2(a.p_ge.d) || !pow2(a.p_e.d) || !pow2(a.p_run.d))
-    return false;
+  if (a.chain_code == kChainGeneric)
+    return kPermuteGeneral;
+  const int body = pow2(a.p_ge.d) && pow2(a.p_e.d) && pow2(a.p_run.d) && a.p_m % a.p_t == 0
+                       ? kPermuteShift
+                       : kPermuteDiv;
   // the direct kernel takes a batch entry's offsets from the innermost level
   for (int j = 0; j + 1 < kBatchLevels; ++j)
     if (a.lv[j].div.d != 1 || a.lv[j].vcnt != 1)
-      return false;
+      return kPermuteGeneral;
   const int k = chain_param_stage(a.chain_code);
   if (k < 0)
-    return true;
+    return body;
   const DevStage &s = a.chain.st[k];
   if (s.vec != 0)
-    return false;
+    return kPermuteGeneral;
   if (s.mode == kChanNone)
-    return true;
+    return body;
   const int64_t plane = C * M * E;
   if (s.mode != kChanDim || s.ch_rs != M * E || s.ch_re != C || a.dbase % plane >= M * E)
-    return false;
+    return kPermuteGeneral;
   for (int j = 0; j < kBatchLevels; ++j)
     if (a.lv[j].div.d > 1 && a.lv[j].ds % plane != 0)
-      return false;
+      return kPermuteGeneral;
   a.p_cmask = ~0u;
-  return true;
+  return body;
 }
 
 // Valid source columns [lo, hi) of a box along the innermost axis.
@@ -1101,14 +1153,17 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
     for (int j = 0; j < n; ++j)
       a.lv[kBatchLevels - n + j] = axis_level(a, b, idx[j], 1);
     const int64_t E = a.vext[r - 1], C = a.vext[r - 3], M = a.vext[r - 2], T = a.p_t;
-    a.p_tiles = make_div(b.ext[r - 2] / T);
+    a.p_m = static_cast<uint32_t>(b.ext[r - 2]);
+    a.p_tiles = make_div(ceil_div(b.ext[r - 2], T));
     a.p_cgt = make_div(work / (C / a.p_g));
     a.p_ce = make_div(C * E);
     a.p_ge = make_div(int64_t{a.p_g} * E);
     a.p_e = make_div(E);
     a.p_run = make_div(T * E * a.wout / 16);
     a.p_dsc = M * E;
-    a.p_direct = permute_direct(a, C, M, E) ? 1 : 0;
+    a.p_direct = permute_direct(a, C, M, E);
+    if (a.p_direct == kPermuteGeneral && a.p_m % T)
+      fail("internal_launch_check", "a cut m-tile outside the direct permute");
     break;
   }
   case kFamInterleave:
@@ -1535,10 +1590,14 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
     // a direct launch replaces each division by a shift and mask, and each
     // vector's parameter entry by c & p_cmask
     const int pk = chain_param_stage(a.chain_code);
-    if (a.p_direct) {
+    const int64_t M = a.p_m;
+    if (int64_t{a.p_tiles.d} != ceil_div(M, T) || (M % T && a.p_direct != kPermuteDiv))
+      bad_launch(dp, "m-tiles disagree with the box");
+    if (a.p_direct == kPermuteShift)
       for (const FastDiv *f : {&a.p_ge, &a.p_e, &a.p_run})
         if (!pow2(f->d) || f->m != 1 || (uint64_t{1} << f->s) != f->d)
           bad_launch(dp, "a direct permute divides by a number that is not a power of two");
+    if (a.p_direct) {
       if (a.chain_code == kChainGeneric || (pk >= 0 && a.chain.st[pk].vec != 0) ||
           (a.p_cmask != 0 && a.p_cmask != ~0u))
         bad_launch(dp, "a direct permute with a chain it cannot run");
@@ -1559,7 +1618,8 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
       int64_t sbase = a.sbase, dbase = a.dbase;
       if (decompose_rt(kBatchLevels, a.lv, batch, sbase, dbase))
         bad_launch(dp, "a permute block reaches a pad");
-      for (int64_t tt = 0; tt < T; ++tt) {
+      const int64_t rows = std::min(T, M - m0);
+      for (int64_t tt = 0; tt < rows; ++tt) {
         const int64_t so = sbase + (m0 + tt) * CE + int64_t{cg} * GE;
         ck.src_run(so, GE, false);
         if ((so * win) % 16 != 0)
@@ -1567,10 +1627,10 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
       }
       for (int64_t cl = 0; cl < G; ++cl) {
         const int64_t c = int64_t{cg} * G + cl;
-        ck.dst_run(dbase + c * a.p_dsc + m0 * E, T * E, false);
+        ck.dst_run(dbase + c * a.p_dsc + m0 * E, rows * E, false);
         if (((dbase + c * a.p_dsc + m0 * E) * wout) % 16 != 0)
           bad_launch(dp, "unaligned destination runs");
-        for (int64_t tt = 0; tt < T; ++tt)
+        for (int64_t tt = 0; tt < rows; ++tt)
           for (int64_t e = 0; e < E; e += VI) {
             const int64_t o = dbase + c * a.p_dsc + (m0 + tt) * E + e;
             ck.channels(o, VI);

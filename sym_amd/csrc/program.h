@@ -225,7 +225,8 @@ struct KArgs {
   uint32_t p_g, p_pad2_; // G
   // direct launches (p_direct): a vector's parameter entry is c & p_cmask
   // (~0: the stage is per channel along c; 0: per tensor)
-  uint32_t p_cmask, p_pad_;
+  uint32_t p_cmask;
+  uint32_t p_m;         // m of the box
   int64_t p_dsc;        // destination stride of c (M*E)
   Chain chain;
   // ragged transpose: extents of q and c in the box (the last tile along
@@ -249,9 +250,7 @@ struct KArgs {
   int32_t res_rank;
   int32_t family;    // Family of this launch (a program's edge boxes may take
                      // another one than its whole tiles or vectors)
-  int32_t p_direct;  // permute: G*E, E and the run are powers of two, one
-                     // batch level, and the parameter stage's channel is c
-                     // or 0 (permute_direct)
+  int32_t p_direct;  // permute: PermuteBody of the launch (permute_direct)
   int64_t work64;    // generic: elements of the box
   uint64_t fill64;
   int64_t pext[kMaxRank]; // padded extents
@@ -264,6 +263,11 @@ struct KArgs {
   int64_t rs[kMaxRank]; // result strides and extents (channel expressions)
   int64_t re[kMaxRank];
 };
+
+// How a permute launch runs: the general kernel, or the direct one (one batch
+// level, the parameter stage's channel c or 0) with shifts (G*E, E and a run
+// are powers of two, T divides the box's m) or with divisions.
+enum PermuteBody : int32_t { kPermuteGeneral = 0, kPermuteShift = 1, kPermuteDiv = 2 };
 
 // Arguments of a direct permute launch (KArgs::p_direct): only the fields its
 // blocks read, 34 dwords that a block fetches in one round of scalar loads.
@@ -290,6 +294,8 @@ struct PermArgs {
   uint32_t nout;                      // 16-byte vectors a block stores
   uint32_t cmask;                     // a vector's parameter entry: c & cmask
   uint32_t scale_off, zp_off, zp_per_ch;
+  uint32_t ge_d, ge_m, e_d, e_m, run_d, run_m; // kPermuteDiv: FastDivs (shifts above)
+  uint32_t m;                                  // kPermuteDiv: m of the box
 };
 
 // Row gather of an indexed plan (index_select along axis 0, at most one cast):

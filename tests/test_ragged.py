@@ -125,7 +125,25 @@ def image_cases(case):
         yield "%s %s %s" % (dtype, shape, [type(o).__name__ for o in ops]), plan.blob, _source(shape, dtype, rng)
 
 
+# [B, S, H, D] -> [B, H, S, D]: heads and head dims whose blocks are no power
+# of two, and sequence lengths that cut the last block of rows
+PERMUTES = [(2, 5, 12, 64), (1, 7, 40, 128), (3, 13, 32, 96), (2, 9, 8, 128), (1, 333, 16, 64), (2, 2, 6, 32)]
+
+
+def permute_cases(shape):
+    rng = np.random.default_rng(sum(shape))
+    out = [shape[i] for i in (0, 2, 1, 3)]
+    for axis in (None, 1, 2):
+        for dtype, ops in _chains(out, axis, rng):
+            if axis is not None and not any(isinstance(o, (EN.Dequantize, EN.Quantize)) for o in ops):
+                continue
+            plan = EN.encode(list(shape), dtype, [EN.Transpose((0, 2, 1, 3))] + ops)
+            yield "%s %s axis %s %s" % (dtype, shape, axis, [type(o).__name__ for o in ops]), plan.blob, \
+                _source(shape, dtype, rng)
+
+
 GROUPS = [("transpose", c, transpose_cases) for c in TRANSPOSES]
+GROUPS += [("permute", c, permute_cases) for c in PERMUTES]
 GROUPS += [("image", c, image_cases) for c in IMAGES]
 GROUPS += [("rows", c, rows_cases) for c in ROWS]
 GROUPS += [("flat", c, flat_cases) for c in FLAT]
