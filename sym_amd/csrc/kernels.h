@@ -70,11 +70,11 @@ __device__ __forceinline__ float op_f16_f32_value(uint32_t h) {
   return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<unsigned short>(h)));
 }
 
+// Round to nearest even in 32 bits (without NaNs the sum cannot wrap); a NaN
+// keeps its upper payload, quieted.
 __device__ __forceinline__ uint32_t op_f32_bf16(uint32_t b) {
-  if ((b & 0x7fffffffu) > 0x7f800000u)
-    return ((b >> 16) | 0x40u) & 0xffffu;
-  const uint64_t w = b;
-  return static_cast<uint32_t>((w + 0x7fffu + ((w >> 16) & 1u)) >> 16);
+  const uint32_t r = (b + 0x7fffu + ((b >> 16) & 1u)) >> 16;
+  return (b & 0x7fffffffu) > 0x7f800000u ? (b >> 16) | 0x40u : r;
 }
 
 // symmetric_rne: t = fl32(x * inv); maxNum(t, -128) then minNum(t, 127)
@@ -496,6 +496,14 @@ __device__ __forceinline__ void chain_vec(const KArgs &a, uint32_t (&v)[V], int6
     }
   } else if constexpr (CH == kChainQuant) {
     stage_vec<V, CUT>(a, a.chain.st[0], v, o);
+  } else if constexpr (CH == kChainF32BF16) {
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+      v[e] = op_f32_bf16(v[e]);
+  } else if constexpr (CH == kChainBF16F32) {
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+      v[e] <<= 16;
   } else {
 #pragma unroll
     for (int k = 0; k < kMaxStages; ++k) {
@@ -1253,6 +1261,10 @@ __device__ __forceinline__ void chain_vec_direct(uint32_t (&v)[V], const VecPara
       v[e] = quant_value(op_f16_f32_value(v[e]), p.sc);
     else if constexpr (CH == kChainQuant)
       v[e] = op_quant(v[e], p.sc);
+    else if constexpr (CH == kChainF32BF16)
+      v[e] = op_f32_bf16(v[e]);
+    else if constexpr (CH == kChainBF16F32)
+      v[e] <<= 16;
   }
 }
 
@@ -1619,6 +1631,14 @@ hipError_t interleave_launch(const KArgs &a, hipStream_t s) {
     case kChainQuant:                                                                      \
       if (w == 33)                                                                         \
         return FN<4, 1, kChainQuant>(a, s);                                                \
+      break;                                                                               \
+    case kChainF32BF16:                                                                    \
+      if (w == 34)                                                                         \
+        return FN<4, 2, kChainF32BF16>(a, s);                                              \
+      break;                                                                               \
+    case kChainBF16F32:                                                                    \
+      if (w == 20)                                                                         \
+        return FN<2, 4, kChainBF16F32>(a, s);                                              \
       break;                                                                               \
     default:                                                                               \
       break;                                                                               \

@@ -588,6 +588,10 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
       chain_code = kChainF16Quant;
     else if (ops == V8{kOpQuantize})
       chain_code = kChainQuant;
+    else if (ops == V8{kOpF32toBF16})
+      chain_code = kChainF32BF16;
+    else if (ops == V8{kOpBF16toF32})
+      chain_code = kChainBF16F32;
   }
   if (widths_ok && dense && !needs_expr && !any_pad && r >= 3 && r - 3 <= kBatchLevels) {
     // permute: destination [batch..., c, m, e] from a source holding

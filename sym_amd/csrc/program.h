@@ -51,6 +51,8 @@ enum ChainCode : int32_t {
   kChainDeq = 5,      // dequantize
   kChainF16Quant = 6, // cast f16 -> f32 -> quantize
   kChainQuant = 7,    // quantize
+  kChainF32BF16 = 8,  // cast f32 -> bf16
+  kChainBF16F32 = 9,  // cast bf16 -> f32
 };
 
 // Chains whose permute kernel fits eight waves per SIMD (64 VGPRs) without
