@@ -117,6 +117,70 @@ __global__ __launch_bounds__(kBlock) void k_gather(GatherArgs a) {
   }
 }
 
+// Rows that no wide item divides (GatherArgs::row_units): 16-byte items at any
+// alignment. A row's last item is read from the row's last bytes, moved down
+// in registers and stored in at most four pieces. Result rows share lines, so
+// the stores go through the cache (int8 rows of 1001 bytes 29.1 us, streamed
+// 34.3). Which rows come here, measured: indexed.cpp.
+template <int OP, int IW, bool NTL>
+__global__ __launch_bounds__(kBlock) void k_gather_cut(GatherArgs a) {
+  static_assert(OP != kGatherF16F32, "widening rows keep their narrow whole items");
+  constexpr int NBI = 16, NBO = gather_out_bytes(OP, NBI);
+  constexpr int W = OP == kGatherCopy ? 1 : 4; // bytes of a source unit
+  constexpr int V = NBI / W, WO = NBO / V;
+  constexpr int U = gather_items(OP);
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
+  const uint32_t stride = gridDim.x * (kBlock / 64) * (64 * U);
+  asm volatile("" ::"s"(a.table), "s"(a.dst), "s"(a.idx), "s"(a.work), "s"(a.row_items),
+               "s"(a.row_src), "s"(a.row_dst), "s"(a.row_units), "s"(stride));
+  hot(a.per_row);
+  for (uint32_t base = wave * (64 * U) + lane; base < a.work; base += stride) {
+    vec4 in[U];
+    uint32_t r[U], at[U], back[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t i = base + 64u * u < a.work ? base + 64u * u : base;
+      r[u] = fdiv(i, a.per_row);
+      at[u] = (i - r[u] * a.row_items) * V;
+      back[u] = at[u] + V > a.row_units ? at[u] + V - a.row_units : 0u;
+      int64_t row;
+      if constexpr (IW == 4)
+        row = reinterpret_cast<const int32_t *>(a.idx)[r[u]];
+      else
+        row = reinterpret_cast<const int64_t *>(a.idx)[r[u]];
+      in[u] = ldu_n<NBI, NTL>(a.table + row * a.row_src + (at[u] - back[u]) * W);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u > 0 && base + 64u * u >= a.work)
+        break;
+      uint8_t *dst = a.dst + static_cast<int64_t>(r[u]) * a.row_dst + at[u] * WO;
+      if (back[u] == 0) {
+        stu_n<NBO>(dst, convert<OP, NBI>(in[u]));
+      } else {
+        stu_cut(dst, convert<OP, NBI>(down_bytes(in[u], back[u] * W)), (V - back[u]) * WO);
+      }
+    }
+  }
+}
+
+template <int OP> hipError_t gather_cut(const GatherArgs &a, int iw, bool nt, hipStream_t s) {
+  constexpr int U = gather_items(OP);
+  const dim3 grid(grid_for((static_cast<int64_t>(a.work) + U - 1) / U)), block(kBlock);
+  if (iw == 4 && nt)
+    hipLaunchKernelGGL((k_gather_cut<OP, 4, true>), grid, block, 0, s, a);
+  else if (iw == 4)
+    hipLaunchKernelGGL((k_gather_cut<OP, 4, false>), grid, block, 0, s, a);
+  else if (iw == 8 && nt)
+    hipLaunchKernelGGL((k_gather_cut<OP, 8, true>), grid, block, 0, s, a);
+  else if (iw == 8)
+    hipLaunchKernelGGL((k_gather_cut<OP, 8, false>), grid, block, 0, s, a);
+  else
+    return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
 template <int OP, int NBI>
 hipError_t gather_iw(const GatherArgs &a, int iw, bool nt, hipStream_t s) {
   constexpr int U = gather_items(OP);
@@ -151,6 +215,10 @@ hipError_t gather_iw(const GatherArgs &a, int iw, bool nt, hipStream_t s) {
 hipError_t gather_launch(const GatherArgs &a, int op, int nbi, int iw, bool nt, hipStream_t s) {
   if (a.work == 0)
     return hipSuccess;
+  if (a.row_units != 0)
+    return op == kGatherCopy && nbi == 16     ? gather_cut<kGatherCopy>(a, iw, nt, s)
+           : op == kGatherF32F16 && nbi == 16 ? gather_cut<kGatherF32F16>(a, iw, nt, s)
+                                              : hipErrorInvalidValue;
   switch (op) {
   case kGatherCopy:
     switch (nbi) {

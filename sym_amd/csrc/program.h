@@ -318,6 +318,10 @@ struct GatherArgs {
   uint32_t work;
   uint32_t row_items;
   FastDiv per_row; // division by row_items
+  int64_t row_src, row_dst; // bytes of a table row and of a result row
+  // cut rows: elements of a row (copies: bytes), whose last item may be cut; 0
+  // where every item is whole
+  uint32_t row_units;
 };
 
 } // namespace relx

@@ -177,6 +177,7 @@ struct GatherPlan {
   int iw = 4;           // index bytes
   bool nt = false;      // streaming table loads (long rows)
   int64_t row_items = 1;
+  int64_t row_units = 0; // GatherArgs::row_units
 };
 GatherPlan gather_plan(const Bound &b, const void *table, const void *dst);
 // Launches over every selected row; `idx` holds the device indices.

@@ -856,9 +856,9 @@ hipError_t gather_launch(const GatherArgs &a, int op, int nbi, int iw, bool nt, 
   (void)nt;
   if (a.work == 0)
     return hipSuccess;
-  const int nbo = op == kGatherF32F16 ? nbi / 2 : op == kGatherF16F32 ? nbi * 2 : nbi;
+  (void)nbi;
   const int64_t rows = (static_cast<int64_t>(a.work) + a.row_items - 1) / a.row_items;
-  const int64_t row_bytes = static_cast<int64_t>(a.row_items) * nbi;
+  const int64_t row_bytes = a.row_src;
   std::lock_guard<std::mutex> g(g_mu);
   const uintptr_t ix = reinterpret_cast<uintptr_t>(a.idx);
   if (!inside(ix, ix + static_cast<uintptr_t>(rows * iw), Mem::Device, "row gather indices"))
@@ -878,17 +878,15 @@ hipError_t gather_launch(const GatherArgs &a, int op, int nbi, int iw, bool nt, 
       s, "row gather",
       {{t + static_cast<uintptr_t>(lo * row_bytes), t + static_cast<uintptr_t>((hi + 1) * row_bytes)},
        {ix, ix + static_cast<uintptr_t>(rows * iw)}},
-      {d, d + static_cast<uintptr_t>(static_cast<int64_t>(a.work) * nbo)},
-      [k, op, nbi, nbo, iw] {
-        for (uint32_t i = 0; i < k.work; ++i) {
-          const uint32_t r = i / k.row_items, j = i - r * k.row_items;
+      {d, d + static_cast<uintptr_t>(rows * a.row_dst)},
+      [k, op, rows, iw] {
+        for (int64_t r = 0; r < rows; ++r) {
           const int64_t row = iw == 8 ? reinterpret_cast<const int64_t *>(k.idx)[r]
                                       : reinterpret_cast<const int32_t *>(k.idx)[r];
-          const uint8_t *from = k.table + (row * k.row_items + j) * nbi;
           if (op == kGatherCopy)
-            std::memcpy(k.dst + static_cast<int64_t>(i) * nbo, from, static_cast<size_t>(nbi));
+            std::memcpy(k.dst + r * k.row_dst, k.table + row * k.row_src, static_cast<size_t>(k.row_src));
           else
-            std::memset(k.dst + static_cast<int64_t>(i) * nbo, 0, static_cast<size_t>(nbo));
+            std::memset(k.dst + r * k.row_dst, 0, static_cast<size_t>(k.row_dst));
         }
       }));
 }

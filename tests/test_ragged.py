@@ -202,3 +202,42 @@ def test_results_on_the_gpu(group):
             ctx.execute_d2h(b, dev.data_ptr(), dev.numel(), host.ctypes.data, n, chunk_bytes=4096,
                             source_pinned=0, caller_stream=stream)
             assert host.tobytes() == want, (name, "d2h")
+
+
+# (table dtype, result dtype, row elements): rows of one 16-byte item, of one
+# element more and less than items, and on either side of each length from
+# which rows move in cut items
+GATHERS = [("int8", "int8", (15, 16, 17, 31, 33, 127, 1001)), ("float16", "float16", (7, 8, 9, 17, 63, 501)),
+           ("float32", "float32", (5, 31, 32, 33, 63, 1001)), ("float32", "float16", (7, 8, 9, 11, 33, 1001)),
+           ("float16", "float32", (3, 9, 33, 501))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("src,dst,widths", GATHERS, ids=["%s-%s" % g[:2] for g in GATHERS])
+def test_row_gathers_on_the_gpu(src, dst, widths):
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(len(widths))
+    with P.Context(0) as ctx:
+        for d in widths:
+            rows, count = 211, 333
+            x = _source((rows, d), src, rng)
+            idx = rng.integers(0, rows, count).astype("<i8")
+            idx[:2] = (rows - 1, 0)
+            blob = EN.encode_index_select([rows, d], src, count, "int64", dst)
+            b = P.bind_indexed(P.load_indexed_plan(blob), {}, ("int64", [count], idx.tobytes()))
+            with np.errstate(all="ignore"):
+                want = (O.narrow_f32_f16_bits(x.view(np.uint32)) if (src, dst) == ("float32", "float16") else
+                        O.widen_f16_f32_bits(x.view(np.uint16)) if src != dst else x)[idx].tobytes()
+            sw, rw = x.itemsize, len(want) // (count * d)
+            for shift in (0, 1):
+                print("[gpu-case]", src, dst, d, "shift", shift, flush=True)
+                table = torch.zeros(x.nbytes + 64, dtype=torch.uint8, device="cuda")
+                table[shift * sw:shift * sw + x.nbytes].copy_(torch.from_numpy(x.view(np.uint8).reshape(-1)))
+                out = torch.full((len(want) + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+                ctx.index_select_device(b, table.data_ptr() + shift * sw, x.nbytes,
+                                        out.data_ptr() + shift * rw, len(want),
+                                        stream=torch.cuda.current_stream().cuda_stream)
+                torch.cuda.synchronize()
+                got = out.cpu().numpy()
+                assert got[shift * rw:shift * rw + len(want)].tobytes() == want, (src, dst, d, shift)
+                assert (got[:shift * rw] == 0xA5).all() and (got[shift * rw + len(want):] == 0xA5).all()
