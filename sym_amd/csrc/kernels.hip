@@ -36,6 +36,16 @@ hipError_t launch_box(int family, const KArgs &a, int32_t *status, hipStream_t s
   case kFamPermute:
     e = permute_fast(a, s, handled);
     return handled ? e : permute_generic(a, s);
+  case kFamElement: {
+    const dim3 grid(grid_for((static_cast<int64_t>(a.work) + 3) / 4)), block(kBlock);
+    if (a.nlev == 2)
+      hipLaunchKernelGGL((k_element<2>), grid, block, 0, s, a, status);
+    else if (a.nlev == 4)
+      hipLaunchKernelGGL((k_element<4>), grid, block, 0, s, a, status);
+    else
+      hipLaunchKernelGGL((k_element<8>), grid, block, 0, s, a, status);
+    return hipGetLastError();
+  }
   default:
     hipLaunchKernelGGL(k_generic, dim3(grid_for(a.work64)), dim3(kBlock), 0, s, a, status);
     return hipGetLastError();

@@ -362,8 +362,12 @@ void ragged_policy(KArgs &a, int64_t bytes) {
 // as one ragged launch.
 constexpr int64_t kRaggedWholeElements = int64_t{1} << 14;
 
-// Shortest q and c extents that take the ragged transpose's tiles.
-constexpr int64_t kRaggedMinExtent = 16;
+// The ragged transpose needs one vector of q and takes c extents from here on:
+// a tile is 64 c wide whatever c is, and the element-wise kernel's stores are
+// then the better ones (f32 [64,3,50177] -> f16 [64,50177,3] 32 us element-wise,
+// 55 in tiles; [32,6,20001] 17.4 and 14.1, [32,12,20001] 27.3 and 14.3; along
+// q, [32,20001,4] 15.0 and 12.6, [32,20001,12] 40.8 and 13.1).
+constexpr int64_t kRaggedMinC = 6;
 
 // A chain that a direct permute of planes of `rs` elements and C channels can
 // run: a compile-time one whose parameter stage is per tensor or along c.
@@ -704,7 +708,7 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
       for (int i = 0; i < r - 1; ++i)
         if (a.ss[i] == 1 && a.vext[i] > 1)
           qa = i;
-      if (qa < 0 || a.vext[qa] < kRaggedMinExtent || a.vext[r - 1] < kRaggedMinExtent)
+      if (qa < 0 || a.vext[qa] < 16 / win || a.vext[r - 1] < kRaggedMinC)
         return false;
       a.t_wq = a.t_wc = kRaggedTile; // boxes start at multiples (large tiles: any start)
       int64_t tiles = ceil_div(a.vext[qa], a.t_wq) * ceil_div(a.vext[r - 1], a.t_wc);
@@ -938,6 +942,37 @@ int64_t box_elements(const Box &b, int rank) {
   return n;
 }
 
+// The element-wise launch of box b, whose box_lo and box_ext are set: in 32
+// bits where its elements, the offsets its axes reach and the result offsets
+// its channels divide allow.
+void element_args(const DeviceProgram &dp, const Box &b, KArgs &a) {
+  const int r = a.rank;
+  a.work64 = box_elements(b, r);
+  a.work = 0;
+  a.family = kFamGeneric;
+  int64_t ss = 0, ds = 0;
+  for (int i = 0; i < r; ++i) {
+    ss += (b.ext[i] - 1) * a.ss[i];
+    ds += (b.ext[i] - 1) * a.ds[i];
+  }
+  bool channels = true;
+  for (int k = 0; k < a.chain.n; ++k)
+    channels = channels && (a.chain.st[k].mode != kChanDim || dp.dst_elems < (int64_t{1} << 32));
+  if (a.work64 >= kMaxLaunchWork || std::max(ss, ds) >= kMaxLaunchWork || !channels)
+    return;
+  a.family = kFamElement;
+  a.work = static_cast<uint32_t>(a.work64);
+  a.nlev = r <= 2 ? 2 : r <= 4 ? 4 : 8;
+  a.sbase = a.dbase = 0;
+  for (int i = 0; i < kMaxRank; ++i)
+    a.lv[i] = trivial_level();
+  for (int i = 0; i < r; ++i) {
+    a.lv[a.nlev - r + i] = axis_level(a, b, i, 1);
+    a.sbase += (b.lo[i] - a.lo[i]) * a.ss[i];
+    a.dbase += b.lo[i] * a.ds[i];
+  }
+}
+
 // Arguments of an edge box: the element-wise kernel over the box.
 KArgs edge_args(const DeviceProgram &dp, const Box &b) {
   KArgs a = dp.base;
@@ -945,9 +980,7 @@ KArgs edge_args(const DeviceProgram &dp, const Box &b) {
     a.box_lo[i] = b.lo[i];
     a.box_ext[i] = b.ext[i];
   }
-  a.work64 = box_elements(b, a.rank);
-  a.work = 0;
-  a.family = kFamGeneric;
+  element_args(dp, b, a);
   return a;
 }
 
@@ -1039,6 +1072,8 @@ void valid_columns(const DeviceProgram &dp, const Box &b, int64_t &lo, int64_t &
 // `family`: the program's own, or kFamRaggedTranspose for a box of a
 // transpose program whose last tiles are cut.
 KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
+  if (family == kFamGeneric)
+    return edge_args(dp, b);
   KArgs a = dp.base;
   const int r = a.rank;
   for (int i = 0; i < r; ++i) {
@@ -1179,11 +1214,10 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
     a.i_loc = static_cast<int32_t>(a.lo[r - 1]);
     a.i_vc = static_cast<int32_t>(a.vext[r - 1]);
     break;
-  default: {
-    work = box_elements(b, r);
+  default:
+    break;
   }
-  }
-  a.work = family == kFamGeneric ? 0 : static_cast<uint32_t>(work);
+  a.work = static_cast<uint32_t>(work);
   a.work64 = family == kFamFlat ? b.ext[0] : work; // a flat box may be a tail alone
   return a;
 }
@@ -1647,6 +1681,9 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
     break;
   }
   default: {
+    const bool element = dp.family == kFamElement;
+    if (element && (a.work64 >= kMaxLaunchWork || a.work != a.work64))
+      bad_launch(dp, "work above 2^31");
     for (int64_t i = 0; i < a.work64; ++i) {
       int64_t rem = i, dof = 0, sof = 0;
       bool pad = false;
@@ -1663,6 +1700,17 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
       ck.dst_run(dof, 1, false);
       if (!pad)
         ck.src_run(sof, 1, false);
+      if (element) { // the kernel's own arithmetic gives the same element
+        int64_t s32 = a.sbase, d32 = a.dbase;
+        const bool p32 = decompose_rt(a.nlev, a.lv, static_cast<uint32_t>(i), s32, d32);
+        if (p32 != pad || d32 != dof || (!pad && s32 != sof))
+          bad_launch(dp, "the levels disagree with the box");
+        for (int k = 0; k < a.chain.n; ++k) {
+          const DevStage &s = a.chain.st[k];
+          if (s.mode == kChanDim && chan_of(s, dof) != (dof / s.ch_rs) % s.ch_re)
+            bad_launch(dp, "a 32-bit channel disagrees with its map");
+        }
+      }
     }
   }
   }
@@ -1697,13 +1745,12 @@ int64_t launch_all(const DeviceProgram &dp, std::vector<KArgs> launches, const v
                        reinterpret_cast<uintptr_t>(dst) % 16 == 0;
   int64_t n = 0;
   for (KArgs &a : launches) {
-    if (!aligned && a.family != kFamGeneric && a.family != kFamRaggedTranspose &&
-        a.family != kFamRows && a.family != kFamRaggedInterleave) {
-      a.family = kFamGeneric;
-      int64_t e = 1;
-      for (int i = 0; i < a.rank; ++i)
-        e *= a.box_ext[i];
-      a.work64 = e;
+    if (!aligned && (a.family == kFamStream || a.family == kFamFlat || a.family == kFamTranspose ||
+                     a.family == kFamInterleave || a.family == kFamPermute)) {
+      Box b{};
+      std::copy(a.box_lo, a.box_lo + a.rank, b.lo);
+      std::copy(a.box_ext, a.box_ext + a.rank, b.ext);
+      element_args(dp, b, a);
     }
     if (verify_enabled())
       verify_launch(dp, a, wire_lo, wire_hi);

@@ -114,6 +114,7 @@ enum Family : int32_t {
   kFamRaggedTranspose = 5, // batched 2-D transpose of any extents and row alignments
   kFamRows = 6, // innermost axis contiguous on both sides, rows of any length, alignment and pads
   kFamRaggedInterleave = 8, // planar -> interleaved, any pixel count and plane alignment
+  kFamElement = 9, // element-wise in 32 bits: a generic box below 2^31 elements and offsets
   kFamFlat = 7, // one contiguous axis whose channels or length fit no whole vectors
 };
 

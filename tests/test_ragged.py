@@ -48,7 +48,11 @@ def _source(shape, dtype, rng):
 # (rows, cols) [batch] around the tile widths: one row of a vector less or
 # more than a tile, extents of the smallest tile launch, several tiles
 TRANSPOSES = [(None, 16, 16), (None, 17, 31), (None, 63, 65), (None, 64, 130), (None, 129, 127),
-              (None, 257, 190), (3, 33, 67), (2, 128, 129)]
+              (None, 257, 190), (3, 33, 67), (2, 128, 129),
+              # either side of the smallest c and q that take tiles; the others
+              # run element-wise
+              (None, 5, 40), (None, 6, 40), (2, 40, 3), (None, 130, 4), (None, 70, 7), (None, 70, 8),
+              (2, 35, 15)]
 
 
 def transpose_cases(case):
@@ -142,7 +146,35 @@ def permute_cases(shape):
                 _source(shape, dtype, rng)
 
 
+# Plans that no vector or tile kernel takes (rows and extents below a vector,
+# channel maps along a merged axis, pads beside a transpose), one element at a
+# time: (shape, perm, pads, reshape)
+ELEMENTS = [((3, 5, 2, 7), (2, 0, 3, 1), (), None), ((40, 3), None, ((0, 1, 2), (1, 0, 1)), None),
+            ((9, 33), (1, 0), ((0, 2, 1),), None), ((4, 6, 10), (1, 0, 2), (), (24, 10)),
+            ((2, 3, 2, 3, 2, 3), (5, 3, 1, 4, 2, 0), (), None)]
+
+
+def element_cases(case):
+    shape, perm, pads, to = case
+    rng = np.random.default_rng(sum(shape))
+    for axis in [None] + list(range(len(shape))):
+        for dtype, ops in _chains(shape, axis, rng):
+            if axis is not None and not any(isinstance(o, (EN.Dequantize, EN.Quantize)) for o in ops):
+                continue
+            layout = ([EN.Transpose(perm)] if perm else [])
+            layout += [EN.Pad(a, lo, hi, 3 if dtype == "int8" else 1.5) for a, lo, hi in pads]
+            layout += [EN.Reshape(to)] if to else []
+            ops = layout + ops if axis is None else ops + layout
+            try:
+                plan = EN.encode(list(shape), dtype, ops)
+            except EN.EncodeError:
+                continue
+            yield "%s %s axis %s %s" % (dtype, shape, axis, [type(o).__name__ for o in ops]), plan.blob, \
+                _source(shape, dtype, rng)
+
+
 GROUPS = [("transpose", c, transpose_cases) for c in TRANSPOSES]
+GROUPS += [("element", c, element_cases) for c in ELEMENTS]
 GROUPS += [("permute", c, permute_cases) for c in PERMUTES]
 GROUPS += [("image", c, image_cases) for c in IMAGES]
 GROUPS += [("rows", c, rows_cases) for c in ROWS]
