@@ -749,6 +749,13 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
     for (uint32_t i = k; i < nst; ++i)
       ch.st[i - k].vec = 0;
   dp->family = family;
+  // the fast families prove every channel; so do element-wise stages per tensor
+  // or along a dimension no longer than its table
+  for (uint32_t i = k; i < nst && family == kFamGeneric; ++i) {
+    const HostStage &h = p.stages[i];
+    dp->reports = dp->reports || h.mode == kChanExpr ||
+                  (h.mode == kChanDim && b.result_extents[static_cast<size_t>(h.dim)] > h.len);
+  }
   a.chain_code = chain_code;
   static const char *names[] = {"generic", "stream", "transpose", "interleave", "permute",
                                 "generic", "generic", "generic", "generic"};
@@ -1736,7 +1743,7 @@ int64_t launch_program(const DeviceProgram &dp, int64_t v0, int64_t v1, bool fir
                     part ? v0 * dp.chunk_stride : 0, part ? v1 * dp.chunk_stride : -1);
 }
 
-int64_t launch_all(const DeviceProgram &dp, std::vector<KArgs> launches, const void *src,
+int64_t launch_all(const DeviceProgram &dp, const std::vector<KArgs> &launches, const void *src,
                    void *dst, const float *pf, const int32_t *pi, int32_t *status, hipStream_t s,
                    int64_t wire_lo, int64_t wire_hi) {
   // the fast kernels move 16-byte vectors: buffers that are not 16-byte
@@ -1744,7 +1751,8 @@ int64_t launch_all(const DeviceProgram &dp, std::vector<KArgs> launches, const v
   const bool aligned = reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(dst) % 16 == 0;
   int64_t n = 0;
-  for (KArgs &a : launches) {
+  for (const KArgs &laid : launches) {
+    KArgs a = laid;
     if (!aligned && (a.family == kFamStream || a.family == kFamFlat || a.family == kFamTranspose ||
                      a.family == kFamInterleave || a.family == kFamPermute)) {
       Box b{};

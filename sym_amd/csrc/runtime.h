@@ -67,6 +67,8 @@ struct DeviceProgram {
   int64_t wire_elems = 0, wire_bytes = 0, dst_elems = 0;
   int chunk_axis = -1;
   int64_t chunk_stride = 0, chunk_align = 1;
+  bool reports = false; // a launch may select a channel outside its parameters (element-wise
+                        // kernels set the status flag); else every channel is proven in range
   int qa = -1, ca = -1; // transpose: source-inner (destination row) and destination-inner axes
   std::vector<float> pf;
   std::vector<int32_t> pi;
@@ -91,7 +93,7 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
 int64_t axis_align(const DeviceProgram &dp, int i);
 // Launch boxes (verified first when RELX_VERIFY_LAUNCHES is set, their
 // source reads inside wire elements [wire_lo, wire_hi), wire_hi < 0: all).
-int64_t launch_all(const DeviceProgram &dp, std::vector<KArgs> launches, const void *src,
+int64_t launch_all(const DeviceProgram &dp, const std::vector<KArgs> &launches, const void *src,
                    void *dst, const float *pf, const int32_t *pi, int32_t *status, hipStream_t s,
                    int64_t wire_lo = 0, int64_t wire_hi = -1);
 // Launch the program over valid chunk-axis coordinates [v0, v1) (the whole
@@ -160,6 +162,17 @@ struct BoundHandle {
   };
   std::map<std::pair<int, uint32_t>, DevParams> params; // (device, boundary)
   std::map<int, void *> dev_indices;                     // indexed plans, per device
+  // Whole-box launches of a program, laid out on its first device-resident
+  // call, and the parameter block a context gave it (by the context's serial
+  // number, which no later context takes; the latest few).
+  std::map<uint32_t, std::vector<KArgs>> whole;
+  struct ContextParams {
+    uint64_t context;
+    uint32_t boundary;
+    DevParams par;
+  };
+  std::vector<ContextParams> context_params;
+  const std::vector<KArgs> &whole_launches(uint32_t k);
   const DeviceProgram &program(uint32_t k);
   DevParams device_params(int device, uint32_t k);
   // The bound row indices in device memory (int32 when the table has fewer
@@ -277,6 +290,7 @@ struct StaticDevice; // the allocation-free upload's per-device state (below)
 
 struct Context {
   int device = 0;
+  uint64_t serial = 0; // unique in the process
   hipStream_t copies[kCopyStreams] = {};
   hipStream_t compute = nullptr;
   // The stream of chunk `chunk` when a call spreads its chunks over `ns`
@@ -364,6 +378,8 @@ struct StaticDevice {
 // call with `device` current.
 StaticDevice &static_device(int device);
 
+// Entries of BoundHandle::context_params.
+constexpr size_t kBoundContexts = 4;
 // Bounds of Context::param_cache.
 constexpr size_t kParamCacheEntries = 4096;
 constexpr size_t kParamCacheBytes = size_t{16} << 20;
