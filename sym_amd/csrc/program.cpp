@@ -1163,6 +1163,8 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
       a.t_nc = make_div(nc);
       a.t_full = static_cast<uint32_t>(full);
       a.t_flags = (bytes && !wide ? kTileXcd : 0u) | (wide ? kTileSkew : 0u);
+      if (a.win > a.wout && box_elements(b, r) * a.win <= kKeepBytes)
+        a.t_flags |= kTileKeep;
       a.t_choff = 0;
       if (a.t_wc == 128 && row_channel(a, b, dp.qa, dp.ca)) {
         a.t_flags |= kTileRowChannel;
@@ -1438,7 +1440,8 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
     const int VO = 16 / wout;
     const int64_t TQ = a.t_wq, TC = a.t_wc;
     if (!(TQ == 64 || (TQ == 128 && win == 1)) || !(TC == 64 || (TC == 128 && TQ == 128)) ||
-        a.t_nc.d != a.t_group.d / a.t_g.d || (a.t_flags & ~(kTileXcd | kTileSkew | kTileRowChannel | kTileZeroPoint0)) ||
+        a.t_nc.d != a.t_group.d / a.t_g.d || (a.t_flags & ~(kTileXcd | kTileSkew | kTileRowChannel | kTileZeroPoint0 | kTileKeep)) ||
+        ((a.t_flags & kTileKeep) && win <= wout) ||
         ((a.t_flags & kTileSkew) && (a.t_flags & kTileXcd)) || (TC == 128 && (a.t_flags & kTileXcd)) ||
         ((a.t_flags & kTileRowChannel) && TC != 128))
       bad_launch(dp, "tile geometry disagrees with the kernel");

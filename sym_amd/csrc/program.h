@@ -162,6 +162,10 @@ constexpr uint32_t kTileRowChannel = 4;
 // dequantization), so the kernel leaves the subtraction out.
 constexpr uint32_t kTileZeroPoint0 = 8;
 
+// A narrowing transpose whose source is at most kKeepBytes: half the 256 MB
+// Infinity Cache.
+constexpr uint32_t kTileKeep = 64;
+constexpr int64_t kKeepBytes = int64_t{128} << 20;
 // Ragged transposes: streaming loads, streaming stores.
 constexpr uint32_t kTileNtLoad = 16;
 constexpr uint32_t kTileNtStore = 32;
