@@ -639,7 +639,7 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
   if (family == kFamGeneric && widths_ok && dense && !needs_expr) {
     // stream: innermost axis contiguous on both sides, unpadded
     // a single contiguous axis need not be a multiple of the vector: its
-    // tail (fewer than V elements) runs element-wise (prefix_launches)
+    // launches then run k_flat, which takes the tail too (prefix_launches)
     if (a.ss[r - 1] == 1 && a.ds[r - 1] == 1 && !inner_pad &&
         (a.vext[r - 1] % V == 0 || (r == 1 && a.vext[0] >= V))) {
       bool ok = true;
@@ -672,8 +672,8 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
         if (a.ss[i] == 1 && a.vext[i] > 1)
           qa = i;
       const int VI = 16 / win, VO = 16 / wout;
-      // extents need not be multiples of 64: the launches split off the
-      // partial tiles at the q and c edges and run them element-wise
+      // extents need not be multiples of 64: boxes with cut tiles run as
+      // ragged launches (prefix_launches)
       if (qa >= 0 && a.vext[qa] >= 64 && a.vext[r - 1] >= 64 && a.ss[r - 1] % VI == 0 &&
           a.ds[qa] % VO == 0) {
         bool ok = true;
@@ -1375,6 +1375,23 @@ struct Checker {
       bad_launch(dp, "unaligned " + std::to_string(n * a.wout) +
                          "-byte destination access at element " + std::to_string(off));
   }
+  // The source element that the element-wise map gives dense result offset o
+  // (-1: a pad): what a kernel of another family must read for it.
+  int64_t source_of(int64_t o) const {
+    int64_t s = 0;
+    for (int k = 0; k < a.rank; ++k) {
+      const int64_t v = (o / a.ds[k]) % a.pext[k] - a.lo[k];
+      if (v < 0 || v >= a.vext[k])
+        return -1;
+      s += v * a.ss[k];
+    }
+    return s;
+  }
+  void same_source(int64_t o, int64_t s) const {
+    if (source_of(o) != s)
+      bad_launch(dp, "result element " + std::to_string(o) + " takes source element " +
+                         std::to_string(s) + ", its map gives " + std::to_string(source_of(o)));
+  }
   // channels of V consecutive result elements from dense offset o, as the
   // fast kernels index them (constant, or +1 per element)
   void channels(int64_t o, int V) const {
@@ -1507,6 +1524,8 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
       const int64_t s0 = a.sbase + int64_t{i} * V, d0 = a.dbase + int64_t{i} * V;
       ck.src_run(s0, n, n == V);
       ck.dst_run(d0, n, n == V);
+      ck.same_source(d0, s0);
+      ck.same_source(d0 + n - 1, s0 + n - 1);
       for (int k = 0; k < a.chain.n; ++k) { // the entries k_flat takes
         const DevStage &s = a.chain.st[k];
         const uint32_t o = static_cast<uint32_t>(d0), c0 = chan_of(s, o), re = s.ch_re_div.d;
@@ -1539,6 +1558,8 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
       pad |= col >= a.r_hi || col + V <= a.r_lo;
       const int n = std::min<int>(V, static_cast<int>(a.r_len) - p);
       ck.dst_run(dof, n, a.r_nts && n == V);
+      for (int e = 0; e < n; ++e)
+        ck.same_source(dof + e, pad || col + e < a.r_lo || col + e >= a.r_hi ? -1 : sof + e);
       if (!pad) {
         if (std::abs(at - col) >= V)
           bad_launch(dp, "a vector moves by its whole width");
@@ -1588,6 +1609,8 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
       for (int64_t row = 0; row < qn; ++row) {
         const int64_t d = dbase + (q0 + row) * a.t_dsq + c0;
         ck.dst_run(d, cn, false);
+        for (int64_t c : {int64_t{0}, cn - 1})
+          ck.same_source(d + c, sbase + (c0 + c) * a.t_ssc + q0 + row);
         for (int64_t cv = 0; cv < cn; cv += VO)
           ck.channels(d + cv, static_cast<int>(std::min<int64_t>(VO, cn - cv)));
       }
@@ -1622,6 +1645,11 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
         const int32_t vc = c - a.i_loc;
         if (!pad && static_cast<uint32_t>(vc) < static_cast<uint32_t>(a.i_vc))
           ck.src_run(sbase + vc * a.i_ssc + p0 - back, G, !rag);
+        for (int64_t j : {int64_t{0}, G - back - 1})
+          ck.same_source(dbase + (p0 + j) * CP + c,
+                         pad || static_cast<uint32_t>(vc) >= static_cast<uint32_t>(a.i_vc)
+                             ? -1
+                             : sbase + vc * a.i_ssc + p0 + j);
       }
     }
     break;
@@ -1681,6 +1709,7 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
         for (int64_t tt = 0; tt < rows; ++tt)
           for (int64_t e = 0; e < E; e += VI) {
             const int64_t o = dbase + c * a.p_dsc + (m0 + tt) * E + e;
+            ck.same_source(o, sbase + (m0 + tt) * CE + c * E + e);
             ck.channels(o, VI);
             if (a.p_direct && pk >= 0 &&
                 chan_of(a.chain.st[pk], o) != (static_cast<uint32_t>(c) & a.p_cmask))
@@ -1749,8 +1778,9 @@ int64_t launch_program(const DeviceProgram &dp, int64_t v0, int64_t v1, bool fir
 int64_t launch_all(const DeviceProgram &dp, const std::vector<KArgs> &launches, const void *src,
                    void *dst, const float *pf, const int32_t *pi, int32_t *status, hipStream_t s,
                    int64_t wire_lo, int64_t wire_hi) {
-  // the fast kernels move 16-byte vectors: buffers that are not 16-byte
-  // aligned take the element-wise kernel
+  // these families move aligned 16-byte vectors: with buffers that are not
+  // 16-byte aligned their boxes run element-wise (the ragged ones and the rows
+  // take any alignment)
   const bool aligned = reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(dst) % 16 == 0;
   int64_t n = 0;
