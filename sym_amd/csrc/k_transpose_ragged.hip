@@ -12,11 +12,14 @@
 // Bound by memory: a tile row that starts inside a 128-byte line shares that
 // line with the next tile, so the line is fetched, or written in part, twice
 // unless both tiles run on one XCD at about the same time. Hence the orders
-// and cache policies of ragged_policy (program.cpp). Measured, buffers of
-// three calls in turn: f32 [16,1001,770] -> f16 [16,770,1001] (74 MB) 74.9
-// (element-wise) -> 13.0 us, 5.7 TB/s; int8 [1027,4099] -> f32 (21 MB) 32.7
-// -> 8.5 us; int8 [3637,7047] -> f32 (128 MB) 178 -> 29 us; f32 [262143,64]
-// (134 MB) 96 -> 28 us; int8 [4096,11007] -> f16 (135 MB) 305 -> 24.5 us.
+// and cache policies of ragged_policy (program.cpp). Measured against the
+// element-wise kernel, buffers of three calls in turn: f32 [16,1001,770] ->
+// bf16 [16,770,1001] (74 MB) 74.9 -> 12.9 us, 5.7 TB/s (18.0 from HBM, buffers
+// of twelve calls); int8 [1027,4099] -> f32 (21 MB) 32.7 -> 7.7 us; int8
+// [3637,7047] -> f32 (128 MB) 178 -> 28.5 us; f32 [262143,64] (134 MB) 96 ->
+// 27 us; int8 [4096,11007] -> f16 (135 MB) 305 -> 23.8 us. Reading the
+// arguments in one batch and the parameters beside the tile loads is 1-6% of
+// these.
 #include "kernels.h"
 
 namespace relx {
@@ -39,6 +42,20 @@ template <int TQ, int TC> __device__ __forceinline__ RagTile rag_tile(const KArg
   p.qn = static_cast<int>(min(static_cast<uint32_t>(TQ), a.t_qn - q0));
   p.cn = static_cast<int>(min(static_cast<uint32_t>(TC), a.t_cn - c0));
   return p;
+}
+
+// Every argument a block reads, in one batch of scalar loads (see hot() in
+// kernels.h).
+template <int CH> __device__ __forceinline__ void rag_hot(const KArgs &a) {
+  asm volatile("" ::"s"(a.src), "s"(a.dst), "s"(a.work), "s"(a.sbase), "s"(a.dbase), "s"(a.t_full),
+               "s"(a.t_flags), "s"(a.t_ssc), "s"(a.t_dsq), "s"(a.t_qn), "s"(a.t_cn), "s"(gridDim.x));
+  hot(a.t_plane);
+  hot(a.t_group);
+  hot(a.t_g);
+  hot(a.t_tail);
+  hot(a.t_nc);
+  hot_levels<kBatchLevels>(a);
+  hot_chain<CH>(a);
 }
 
 // The tile's source vectors: lane vid of VPR vectors per row. `back`: how far
@@ -105,6 +122,7 @@ __global__ __launch_bounds__(kBlock) void k_transpose_rag(KArgs a) {
   constexpr int VPRI = TQ / VI, VPRO = TC / VO;
   constexpr int NI = TC * VPRI / kBlock, NO = TQ * VPRO / kBlock;
   static_assert(NI * kBlock == TC * VPRI && NO * kBlock == TQ * VPRO, "whole tiles per block");
+  rag_hot<CH>(a);
   const uint32_t t = (a.t_flags & kTileXcd) ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
   if (t >= a.work)
     return;
@@ -149,17 +167,27 @@ __global__ __launch_bounds__(kBlock) void k_transpose_rag_b(KArgs a) {
   constexpr int VPRI = TQ / 16, NI = TC * VPRI / kBlock;
   constexpr int VO = 16 / WOUT, VPRO = TC / VO;
   constexpr int NO = TQ * VPRO / kBlock;
+  rag_hot<CH>(a);
   const uint32_t t = (a.t_flags & kTileXcd) ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
   if (t >= a.work)
     return;
   const RagTile p = rag_tile<TQ, TC>(a, t);
   vec4 in[NI];
   rag_load<1, VPRI, NI>(a, p, in);
+  const int col = threadIdx.x % VPRO * VO;
+  // the store phase's parameters, in flight with the tile loads where a lane
+  // stores few vectors
+  constexpr bool kEarly = NO <= 4;
+  VecParams early[kEarly ? NO : 1];
+  if constexpr (kEarly) {
+#pragma unroll
+    for (int j = 0; j < NO; ++j)
+      early[j] = fetch_params<CH>(a, p.dbase + (threadIdx.x / VPRO + j * (kBlock / VPRO)) * a.t_dsq + col);
+  }
   rag_to_lds<1, VPRI, NI>(p, in, [&](int row, int col, uint32_t x) {
     tile[col * PT + row] = static_cast<uint8_t>(x);
   });
   __syncthreads();
-  const int col = threadIdx.x % VPRO * VO;
 #pragma unroll 4
   for (int j = 0; j < NO; ++j) {
     const int row = threadIdx.x / VPRO + j * (kBlock / VPRO);
@@ -167,7 +195,11 @@ __global__ __launch_bounds__(kBlock) void k_transpose_rag_b(KArgs a) {
       break;
     const uint8_t *tp = tile + row * PT + col;
     const int64_t dof = p.dbase + row * a.t_dsq + col;
-    const VecParams par = fetch_params<CH>(a, dof);
+    VecParams par;
+    if constexpr (kEarly)
+      par = early[j];
+    else
+      par = fetch_params<CH>(a, dof);
     vec4 w = {0u, 0u, 0u, 0u};
     if constexpr (VO == 16) {
       w = *reinterpret_cast<const vec4 *>(tp);
