@@ -469,7 +469,8 @@ int relx_execute_d2h(relx_ctx *ctx, const relx_bound *bound, const void *src, si
  * the device half of relx_execute_h2d and the unit the kernel roofline is
  * measured on; it replaces the reference's kernel launch wrappers
  * reloc::cuda::* (libreloc/include/reloc/CudaKernels.h:28-122).
- * A program on the element-wise kernel reports a stage channel outside its
+ * A program whose channels its binding does not prove in range (a channel
+ * expression, or a dimension longer than its table) reports one outside its
  * parameters through a status flag of its own; the next
  * relx_ctx_synchronize waits for such launches and fails with
  * "channel_out_of_range" once for all of them. */

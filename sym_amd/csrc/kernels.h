@@ -8,8 +8,14 @@
 // reference's NaN encodings, so results are bit-identical to the reference
 // CPU executor (libreloc/src/TypedExecute.cpp:472-499).
 //
-// Families (chosen on the host, program.cpp):
+// Families (chosen on the host, program.cpp; the ragged ones in files of their
+// own):
 //   generic    one element per thread, any rank/stride/pad/channel map
+//              (k_element in 32 bits where the box allows)
+//   rows, flat k_rows.hip: the stream's axes at any row length, alignment and
+//              pads, and channels that change inside a vector
+//   ragged     k_transpose_ragged.hip, k_interleave_ragged.hip: the 2-D
+//              families at any extents and alignments
 //   stream     innermost axis contiguous on both sides: one vector of
 //              16/min(width) elements per thread (16-byte loads/stores)
 //   transpose  batched 2-D transpose through a 64x64 LDS tile (32-bit

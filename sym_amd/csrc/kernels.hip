@@ -1,7 +1,8 @@
-// kernels.hip - the generic kernel's launch and the family dispatcher.
+// kernels.hip - the element-wise kernels' launch and the family dispatcher.
 // Kernel bodies live in kernels.h; the fast families are instantiated in
 // k_stream_fast.hip, k_stream_generic.hip, k_transpose.hip, k_interleave.hip,
-// k_interleave_generic.hip, k_permute.hip.
+// k_interleave_generic.hip, k_permute.hip, and written and instantiated in
+// k_rows.hip, k_transpose_ragged.hip, k_interleave_ragged.hip.
 #include "kernels.h"
 
 namespace relx {

@@ -310,8 +310,9 @@ struct Context {
   int32_t *status = nullptr; // kStatusSlots flags, one per call in flight,
                              // then kDeviceChecks flags of device-resident calls
   uint32_t status_next = 0; // wraps
-  // Device-resident element-wise launches (relx_relayout_device) run on the
-  // caller's stream and return at once: each takes the next of kDeviceChecks
+  // Device-resident launches that may report a channel
+  // (DeviceProgram::reports; relx_relayout_device) run on the caller's stream
+  // and return at once: each takes the next of kDeviceChecks
   // flags and records check_ev after its launch. The flag is read once that
   // event completes: when the slot comes round again, or at synchronize.
   hipEvent_t check_ev[64] = {};
