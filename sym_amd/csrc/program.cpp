@@ -358,8 +358,11 @@ void ragged_policy(KArgs &a, int64_t bytes) {
   a.t_flags = (xcd ? kTileXcd : 0u) | (cold && xcd ? kTileNtLoad : 0u) | (dst ? kTileNtStore : 0u);
 }
 
-// Aligned boxes of at least this many elements whose last tiles are cut run
-// as one ragged launch.
+// Aligned transpose boxes of at least this many elements whose last tiles are
+// cut run as one ragged launch, and a device-resident call's whatever their
+// size (f32 [128,96] -> f16 transposed 11.0 us a pass as tiles and a strip,
+// 7.0 as one launch; [72,200], with two strips, 14.7 and 7.0). A smaller box
+// of a transfer keeps its whole tiles and strips.
 constexpr int64_t kRaggedWholeElements = int64_t{1} << 14;
 
 // The ragged transpose needs one vector of q and takes c extents from here on:
@@ -1254,7 +1257,7 @@ std::vector<KArgs> axis_launches(const DeviceProgram &dp, int axis, int64_t plo,
 }
 
 std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed, int axis,
-                                   int64_t plo, int64_t phi) {
+                                   int64_t plo, int64_t phi, bool resident) {
   const KArgs &a = dp.base;
   Box b{};
   for (int i = 0; i < a.rank; ++i) {
@@ -1272,9 +1275,9 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
   std::vector<KArgs> out;
   std::vector<Box> edges;
   // A transpose box whose q or c extent is not a multiple of the tile runs
-  // as one ragged launch; a small one keeps its whole tiles on the tile
-  // kernel and runs the strips past them (the q strip over the whole c range,
-  // the c strip beside the whole q tiles) as ragged launches.
+  // as one ragged launch; a transfer's small one keeps its whole tiles on the
+  // tile kernel and runs the strips past them (the q strip over the whole c
+  // range, the c strip beside the whole q tiles) as ragged launches.
   int family = dp.family;
   if (family == kFamStream && a.rank == 1 && b.ext[0] % a.vec != 0)
     family = kFamFlat; // the tail past the last vector in the same launch
@@ -1288,7 +1291,7 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
   if (family == kFamRaggedInterleave && b.ext[a.rank - 2] < a.vec)
     return {edge_args(dp, b)};
   if (family == kFamTranspose && (b.ext[dp.qa] % a.t_wq || b.ext[dp.ca] % a.t_wc)) {
-    if (box_elements(b, a.rank) >= kRaggedWholeElements) {
+    if (resident || box_elements(b, a.rank) >= kRaggedWholeElements) {
       family = kFamRaggedTranspose;
     } else {
       const int q = dp.qa, c = dp.ca;

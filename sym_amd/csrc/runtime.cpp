@@ -271,7 +271,7 @@ const std::vector<KArgs> &BoundHandle::whole_launches(uint32_t k) {
   std::lock_guard<std::mutex> g(mu);
   auto it = whole.find(k);
   if (it == whole.end())
-    it = whole.emplace(k, box_launches(dp, 0, 0, true, true)).first;
+    it = whole.emplace(k, prefix_launches(dp, nullptr, -1, 0, 0, true)).first;
   return it->second;
 }
 
@@ -1550,8 +1550,9 @@ int64_t verify_launches(BoundHandle &h, uint32_t k, int64_t chunk_bytes) {
     schedule_done();
     whole = whole || (dp.chunk_axis >= 0 && p.units > p.per_chunk);
   }
-  if (whole) {
-    for (const KArgs &a : box_launches(dp, 0, 0, true, true)) // the device-resident launch
+  // the device-resident launches, where no schedule above had them
+  if (whole || dp.family == kFamTranspose) {
+    for (const KArgs &a : h.whole_launches(k))
       check(a);
     schedule_done();
   }

@@ -86,9 +86,10 @@ std::vector<KArgs> box_launches(const DeviceProgram &dp, int64_t v0, int64_t v1,
 // (the whole box when axis < 0).
 std::vector<KArgs> axis_launches(const DeviceProgram &dp, int axis, int64_t plo, int64_t phi);
 // Launches for one coordinate of each axis before `axis` (fixed[0..axis))
-// and padded coordinates [plo, phi) of `axis`.
+// and padded coordinates [plo, phi) of `axis`. `resident`: a device-resident
+// call's launches (see kRaggedWholeElements).
 std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed, int axis,
-                                   int64_t plo, int64_t phi);
+                                   int64_t plo, int64_t phi, bool resident = false);
 // Coordinates a box along axis i must keep together (0: never split).
 int64_t axis_align(const DeviceProgram &dp, int i);
 // Launch boxes (verified first when RELX_VERIFY_LAUNCHES is set, their

@@ -273,3 +273,36 @@ def test_row_gathers_on_the_gpu(src, dst, widths):
                 got = out.cpu().numpy()
                 assert got[shift * rw:shift * rw + len(want)].tobytes() == want, (src, dst, d, shift)
                 assert (got[:shift * rw] == 0xA5).all() and (got[shift * rw + len(want):] == 0xA5).all()
+
+
+@pytest.mark.gpu
+def test_a_bound_plan_keeps_no_block_of_a_closed_context():
+    """One bound plan with per-channel parameters run by more contexts than it
+    keeps parameter blocks for, each closed before the next is made, then by
+    two contexts that are open together: every result equals the oracle's."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(5)
+    x = rng.integers(-128, 128, (96, 257), dtype=np.int8)
+    plan = EN.encode([96, 257], "int8", [EN.Dequantize(_scale(257, rng), zero_point=_zp(257, rng), axis=1),
+                                         EN.Cast("float16"), EN.Transpose((1, 0))])
+    want = _want(plan.blob, x)
+    b = P.Bound(P.Plan(plan.blob), {}, {})
+    dev = torch.from_numpy(x.view(np.uint8).reshape(-1).copy()).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(ctx):
+        out = torch.full((len(want),), 0xA5, dtype=torch.uint8, device="cuda")
+        for _ in range(2):
+            ctx.relayout_device(b, dev.data_ptr(), out.data_ptr(), stream=stream)
+        ctx.synchronize()
+        torch.cuda.synchronize()
+        assert out.cpu().numpy().tobytes() == want
+
+    for _ in range(7):
+        with P.Context(0) as ctx:
+            run(ctx)
+            # other parameter blocks of the same size where a freed one was
+            torch.full((4096,), 0x7F, dtype=torch.uint8, device="cuda")
+    with P.Context(0) as first, P.Context(0) as second:
+        for ctx in (first, second, first, second):
+            run(ctx)
