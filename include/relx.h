@@ -159,7 +159,9 @@ typedef struct relx_bound_info {
   int64_t source_extents[RELX_MAX_RANK];
   int result_rank;
   int64_t result_extents[RELX_MAX_RANK];
-  char kernel[32]; /* device kernel family the program runs */
+  char kernel[32]; /* the program's family of whole vectors or tiles ("stream", "transpose",
+                    * "interleave", "permute"), else "generic"; relx_launch_kernels names the
+                    * kernels that its launches run */
   int host_stages_max;  /* leading per-tensor stages a host may apply */
   int host_stages_auto; /* of those, the narrowing ones the host applies by default */
   int64_t wire_bytes_at[RELX_MAX_STAGES + 1]; /* H2D wire (source layout) at boundary k */
@@ -172,9 +174,10 @@ typedef struct relx_bound_info {
   int64_t table_bytes;
   int64_t index_count;
   /* permute programs: 1 when every launch of the whole box (the launches of
-   * relx_relayout_device) runs the direct body, whose divisions are shifts
-   * and whose vectors take stage parameters from their own channel
-   * coordinate; 0 otherwise */
+   * relx_relayout_device) runs the direct body with shifts for its divisions,
+   * whose vectors take stage parameters from their own channel coordinate; 0
+   * otherwise (the direct body with divisions included: relx_launch_kernels
+   * tells it from the general one) */
   int permute_direct;
   /* transpose programs: the q width (source-contiguous axis) of the tile
    * kernel's tiles, 128 for one-byte sources whose q extent is a multiple of
@@ -506,6 +509,20 @@ int relx_host_stage(const relx_bound *bound, int host_stages, const void *src, v
  * set. No counterpart in the reference: it backs this library's tests. */
 int relx_verify_launches(const relx_bound *bound, int wire_boundary, int64_t chunk_bytes,
                          int64_t *launches, relx_err *err);
+
+/* Names of the kernels that relx_relayout_device's launches of this bound
+ * plan run with the wire at `wire_boundary` and 16-byte aligned buffers (an
+ * indexed plan: relx_index_select_device's), each once, separated by commas:
+ * "stream", "flat", "rows", "transpose", "ragged_transpose",
+ * "ragged_transpose_large" (tiles 128 wide), "interleave",
+ * "ragged_interleave", "permute_shift" and "permute_div" (the direct body,
+ * with shifts or divisions), "permute" (the general one), "gather",
+ * "gather_cut", "element" and "generic" (one element at a time, in 32 and in
+ * 64 bits: the slow ones); an empty text when nothing is launched. Buffers
+ * that are not 16-byte aligned run the stream, flat, transpose, interleave and
+ * permute launches element-wise. No counterpart in the reference. */
+int relx_launch_kernels(const relx_bound *bound, int wire_boundary, char *out, size_t out_bytes,
+                        relx_err *err);
 
 /* Block until every call on the context has completed: its own streams, and
  * the device-resident launches that report a status (see

@@ -166,6 +166,7 @@ SIGNATURES = {
     "relx_index_select_device": (_I, [_VP, _VP, _VP, _SZ, _VP, _SZ, _U64, _E]),
     "relx_host_stage": (_I, [_VP, _I, _VP, _VP, _I, _E]),
     "relx_verify_launches": (_I, [_VP, _I, ctypes.c_int64, ctypes.POINTER(ctypes.c_int64), _E]),
+    "relx_launch_kernels": (_I, [_VP, _I, ctypes.c_char_p, _SZ, _E]),
     "relx_ctx_synchronize": (_I, [_VP, _E]),
     "relx_ctx_time_kernels": (_I, [_VP, _I, _E]),
     "relx_ctx_kernel_times": (_I, [_VP, ctypes.POINTER(relx_kernel_times), _E]),

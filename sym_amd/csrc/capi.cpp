@@ -782,6 +782,21 @@ int relx_verify_launches(const relx_bound *bound, int wire_boundary, int64_t chu
   });
 }
 
+int relx_launch_kernels(const relx_bound *bound, int wire_boundary, char *out, size_t out_bytes,
+                        relx_err *err) {
+  return guarded(err, [&] {
+    if (!bound || !out || out_bytes == 0)
+      throw relx::Error("invalid_argument", "null argument");
+    if (wire_boundary < 0)
+      throw relx::Error("invalid_boundary", "negative wire boundary");
+    const std::string s = relx::launch_kernels(const_cast<relx::BoundHandle &>(bound->h),
+                                               static_cast<uint32_t>(wire_boundary));
+    if (s.size() >= out_bytes)
+      throw relx::Error("invalid_argument", "the names need " + std::to_string(s.size() + 1) + " bytes");
+    std::memcpy(out, s.c_str(), s.size() + 1);
+  });
+}
+
 int relx_host_stage(const relx_bound *bound, int host_stages, const void *src, void *wire,
                     int threads, relx_err *err) {
   return guarded(err, [&] {

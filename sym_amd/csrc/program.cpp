@@ -1778,6 +1778,31 @@ int64_t launch_program(const DeviceProgram &dp, int64_t v0, int64_t v1, bool fir
                     part ? v0 * dp.chunk_stride : 0, part ? v1 * dp.chunk_stride : -1);
 }
 
+const char *launch_kernel(const KArgs &a) {
+  switch (a.family) {
+  case kFamStream:
+    return "stream";
+  case kFamFlat:
+    return "flat";
+  case kFamRows:
+    return "rows";
+  case kFamTranspose:
+    return "transpose";
+  case kFamRaggedTranspose:
+    return a.t_wc == kRaggedLargeC ? "ragged_transpose_large" : "ragged_transpose";
+  case kFamInterleave:
+    return "interleave";
+  case kFamRaggedInterleave:
+    return "ragged_interleave";
+  case kFamPermute:
+    return a.p_direct == kPermuteShift ? "permute_shift" : a.p_direct == kPermuteDiv ? "permute_div" : "permute";
+  case kFamElement:
+    return "element";
+  default:
+    return "generic";
+  }
+}
+
 int64_t launch_all(const DeviceProgram &dp, const std::vector<KArgs> &launches, const void *src,
                    void *dst, const float *pf, const int32_t *pi, int32_t *status, hipStream_t s,
                    int64_t wire_lo, int64_t wire_hi) {

@@ -1505,6 +1505,19 @@ KernelBatches kernel_batches(const ChunkPlan &p) {
   return {p.units, n * p.per_chunk, n > 1 ? (chunks - 1) * p.per_chunk : p.units};
 }
 
+std::string launch_kernels(BoundHandle &h, uint32_t k) {
+  if (h.bound->indexed)
+    return h.bound->indices.empty() ? "" : gather_plan(*h.bound, nullptr, nullptr).row_units ? "gather_cut" : "gather";
+  std::vector<std::string> names;
+  for (const KArgs &a : h.whole_launches(k))
+    if (std::find(names.begin(), names.end(), launch_kernel(a)) == names.end())
+      names.push_back(launch_kernel(a));
+  std::string out;
+  for (const std::string &n : names)
+    out += (out.empty() ? "" : ",") + n;
+  return out;
+}
+
 int64_t verify_launches(BoundHandle &h, uint32_t k, int64_t chunk_bytes) {
   const DeviceProgram &dp = h.program(k);
   int64_t n = 0;

@@ -90,6 +90,8 @@ std::vector<KArgs> axis_launches(const DeviceProgram &dp, int axis, int64_t plo,
 // call's launches (see kRaggedWholeElements).
 std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed, int axis,
                                    int64_t plo, int64_t phi, bool resident = false);
+// The kernel that a laid out launch runs (relx_launch_kernels).
+const char *launch_kernel(const KArgs &a);
 // Coordinates a box along axis i must keep together (0: never split).
 int64_t axis_align(const DeviceProgram &dp, int i);
 // Launch boxes (verified first when RELX_VERIFY_LAUNCHES is set, their
@@ -252,6 +254,8 @@ uint32_t auto_host_stages(const BoundHandle &h);
 // (0: both defaults, staged and direct, in each direction) and the whole-box
 // launch of the device-resident path; returns the count.
 int64_t verify_launches(BoundHandle &h, uint32_t k, int64_t chunk_bytes);
+// Kernels of the device-resident launches (relx_launch_kernels).
+std::string launch_kernels(BoundHandle &h, uint32_t k);
 
 // A ROCTX range on the calling thread around one host phase of the pipeline
 // (the reference's TraceRange, libreloc/src/Trace.h:15-39, which its NVTX

@@ -327,7 +327,8 @@ class Bound:
     @property
     def permute_direct(self):
         """True when every whole-box launch of a permute program runs the
-        direct body (shift indexing, parameters by channel coordinate)."""
+        direct body with shifts (parameters by channel coordinate); False for
+        the direct body with divisions too (launch_kernels names it)."""
         return bool(self.info.permute_direct)
 
     @property
@@ -666,6 +667,16 @@ def verify_launches(bound, wire_boundary=0, chunk_bytes=0):
                                     ctypes.byref(n), ctypes.byref(err)):
         _raise(err)
     return n.value
+
+
+def launch_kernels(bound, wire_boundary=0):
+    """Names of the kernels that `bound`'s device-resident launches run with
+    the wire at `wire_boundary` and 16-byte aligned buffers, each once."""
+    err = N.relx_err()
+    out = ctypes.create_string_buffer(256)
+    if N.lib().relx_launch_kernels(bound._h, int(wire_boundary), out, len(out), ctypes.byref(err)):
+        _raise(err)
+    return [n for n in out.value.decode().split(",") if n]
 
 
 def host_stage(bound, host_stages, src_ptr, wire_ptr, threads=8):

@@ -1,0 +1,90 @@
+"""Which kernels each plan's device-resident launches run
+(relx_launch_kernels), for every form of tests/test_ragged.py and
+tests/permute_cases.py: a rule that sent a shape to another kernel than the
+one these files mean to test fails here."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from sym_amd import _native as N
+from sym_amd import encoder as EN
+from sym_amd import pyreloc as P
+from sym_amd import workloads as W
+from tests import permute_cases as PC
+from tests import test_ragged as R
+
+# Per group of test_ragged.py: the kernels that its plans run, every one of
+# them. Parameters that run along neither the rows nor the columns leave the
+# rows and permute-direct kernels; a vector of q or of a pixel group that a
+# wider type does not fill leaves the tile and interleave ones.
+GROUP_KERNELS = {
+    "permute": {"permute_shift", "permute_div", "permute"},
+    "image": {"ragged_interleave", "interleave"},
+    "rows": {"rows", "element"},
+    "flat": {"flat", "stream"},
+}
+
+
+def _kernels(blob, symbols=None, params=None):
+    return P.launch_kernels(P.Bound(P.Plan(blob), symbols or {}, params or {}))
+
+
+@pytest.mark.parametrize("kind", sorted(GROUP_KERNELS))
+def test_kernels_of_the_ragged_groups(kind):
+    seen = set()
+    for k, case, make in R.GROUPS:
+        if k != kind:
+            continue
+        mine = set()
+        for name, blob, _ in make(case):
+            got = _kernels(blob)
+            assert len(got) == 1 and got[0] in GROUP_KERNELS[kind], (name, got)
+            mine.update(got)
+        if kind == "rows":
+            assert "rows" in mine, case
+        seen |= mine
+    assert seen == GROUP_KERNELS[kind]
+
+
+@pytest.mark.parametrize("case", PC.cases(), ids=[c[0] for c in PC.cases()])
+def test_kernels_of_the_permutes(case):
+    """Shifts where every division is one; divisions where only they are
+    missing (24 heads, D = 96); the general body where the parameters do not
+    run along H."""
+    name, blob, _, direct = case
+    want = "permute_shift" if direct else "permute" if " per D" in name or " per S" in name or "batch" in name \
+        else "permute_div"
+    assert _kernels(blob) == [want]
+
+
+def test_random_permutes_take_every_body():
+    assert {_kernels(blob)[0] for _, blob, _ in PC.random_cases(200)} == {"permute_shift", "permute_div", "permute"}
+
+
+def test_kernels_of_the_workloads():
+    assert _kernels(W.c1_plan().blob, {"s0": 64 * 4096}) == ["transpose"]
+    assert _kernels(W.c2_plan(n=3).blob) == ["interleave"]
+    assert _kernels(W.c3_plan().blob, {"s0": 4096, "s1": 11008},
+                    W.param("scale", np.ones(11008, np.float32))) == ["transpose"]
+    assert _kernels(W.c4_plan().blob, {"s0": 512, "s1": 256}, W.param("scale", np.ones(512, np.float32))) == ["stream"]
+    assert _kernels(W.c5_plan().blob, {"B": 2, "S": 64}, W.param("scale", np.ones(32, np.float32))) == ["permute_shift"]
+
+
+def test_kernels_of_a_row_gather():
+    for d, want in ((1024, ["gather"]), (1001, ["gather_cut"])):
+        blob = EN.encode_index_select([64, d], "int8", 8, "int64", "int8")
+        idx = np.arange(8, dtype="<i8")
+        assert P.launch_kernels(P.bind_indexed(P.load_indexed_plan(blob), {}, ("int64", [8], idx.tobytes()))) == want
+
+
+def test_refusals():
+    b = P.Bound(P.Plan(EN.encode([8, 64], "float32", [EN.Cast("float16")]).blob), {}, {})
+    assert P.launch_kernels(b, 0) == ["stream"] and P.launch_kernels(b, 1) == ["stream"]
+    for k in (-1, 2):
+        with pytest.raises(P.BindError, match="invalid_boundary"):
+            P.launch_kernels(b, k)
+    err, out = N.relx_err(), ctypes.create_string_buffer(4)
+    assert N.lib().relx_launch_kernels(b._h, 0, out, 4, ctypes.byref(err)) != 0
+    assert N.lib().relx_launch_kernels(b._h, 0, None, 4, ctypes.byref(err)) != 0
+    assert N.lib().relx_launch_kernels(None, 0, out, 4, ctypes.byref(err)) != 0
