@@ -371,6 +371,18 @@ constexpr int64_t kRaggedWholeElements = int64_t{1} << 14;
 // 55 in tiles; [32,6,20001] 17.4 and 14.1, [32,12,20001] 27.3 and 14.3; along
 // q, [32,20001,4] 15.0 and 12.6, [32,20001,12] 40.8 and 13.1).
 constexpr int64_t kRaggedMinC = 6;
+// Elements a tile must hold on average. A tile costs one block's load, barrier
+// and store whatever it holds, about a nanosecond each with the chip full, so
+// many planes that each fill little of theirs are the element-wise kernel's
+// (f32, tiles and element-wise: [131072,12,12], 144 a tile, 133.7 and 43.4 us;
+// [131072,16,16], 256, 127.3 and 78.5; [2796,6,1000], 375, 72.1 and 39.5;
+// [2796,1000,6], 375, 60.4 and 65.2; [32768,64,8], 512, 37.1 and 42.9;
+// [32768,24,40], 960, 51.1 and 76.6; f16 [65536,16,16] 59.1 and 42.0,
+// [32768,64,8] 30.1 and 39.3). Dequantizing an element at a time costs almost
+// twice as much: int8 -> f16 [174762,6,16], 96 a tile, 164 and 73.5 us;
+// [65536,16,16] 63.3 and 71.0; [13981,6,200], 300, 68.1 and 72.3.
+constexpr int64_t kRaggedTileElements = 384;
+constexpr int64_t kRaggedTileDequantized = 256;
 
 // A chain that a direct permute of planes of `rs` elements and C channels can
 // run: a compile-time one whose parameter stage is per tensor or along c.
@@ -714,11 +726,17 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
       if (qa < 0 || a.vext[qa] < 16 / win || a.vext[r - 1] < kRaggedMinC)
         return false;
       a.t_wq = a.t_wc = kRaggedTile; // boxes start at multiples (large tiles: any start)
-      int64_t tiles = ceil_div(a.vext[qa], a.t_wq) * ceil_div(a.vext[r - 1], a.t_wc);
+      const int64_t plane_tiles = ceil_div(a.vext[qa], a.t_wq) * ceil_div(a.vext[r - 1], a.t_wc);
+      int64_t tiles = plane_tiles;
       for (int i = 0; i < r - 1; ++i)
         if (i != qa)
           tiles *= a.vext[i];
-      if (tiles >= (int64_t{1} << 22) || !row_channels_ok())
+      bool dequantizes = false;
+      for (uint32_t i = k; i < nst; ++i)
+        dequantizes = dequantizes || p.stages[i].op == kOpDequantize;
+      if (tiles >= (int64_t{1} << 22) ||
+          a.vext[qa] * a.vext[r - 1] < plane_tiles * (dequantizes ? kRaggedTileDequantized : kRaggedTileElements) ||
+          !row_channels_ok())
         return false;
       dp->qa = qa;
       dp->ca = r - 1;

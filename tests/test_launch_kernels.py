@@ -17,8 +17,11 @@ from tests import test_ragged as R
 # Per group of test_ragged.py: the kernels that its plans run, every one of
 # them. Parameters that run along neither the rows nor the columns leave the
 # rows and permute-direct kernels; a vector of q or of a pixel group that a
-# wider type does not fill leaves the tile and interleave ones.
+# wider type does not fill, or planes that fill little of a tile, leave the
+# tile and interleave ones.
 GROUP_KERNELS = {
+    "transpose": {"ragged_transpose", "element"},
+    "element": {"element"},
     "permute": {"permute_shift", "permute_div", "permute"},
     "image": {"ragged_interleave", "interleave"},
     "rows": {"rows", "element"},
@@ -43,6 +46,8 @@ def test_kernels_of_the_ragged_groups(kind):
             mine.update(got)
         if kind == "rows":
             assert "rows" in mine, case
+        if kind == "transpose" and case[1] * case[2] >= 500 and min(case[1:]) >= 9:
+            assert mine == {"ragged_transpose"} or case == (2, 35, 15), case
         seen |= mine
     assert seen == GROUP_KERNELS[kind]
 
@@ -60,6 +65,32 @@ def test_kernels_of_the_permutes(case):
 
 def test_random_permutes_take_every_body():
     assert {_kernels(blob)[0] for _, blob, _ in PC.random_cases(200)} == {"permute_shift", "permute_div", "permute"}
+
+
+DEQ = EN.Dequantize(EN.InlineParam((0.03125,)))
+F16 = EN.Cast("float16")
+# Transposes of the last two axes: tiles from 384 elements each on average
+# (256 where an element is dequantized), one vector of q and six c.
+TRANSPOSES = [((64, 12, 12), "float32", [], "element"), ((64, 16, 16), "float32", [], "element"),
+              ((64, 16, 24), "float32", [], "ragged_transpose"), ((64, 16, 23), "float32", [F16], "element"),
+              ((64, 24, 40), "float32", [], "ragged_transpose"), ((64, 6, 640), "float16", [], "ragged_transpose"),
+              ((64, 6, 641), "float16", [], "element"), ((64, 1000, 6), "float32", [], "element"),
+              ((64, 9, 6), "float32", [], "element"), ((64, 6, 16), "int8", [], "element"),
+              ((64, 16, 16), "int8", [DEQ, F16], "ragged_transpose"), ((64, 15, 17), "int8", [DEQ], "element"),
+              ((64, 16, 16), "int8", [], "element"), ((64, 5, 640), "int8", [DEQ], "element"),
+              ((64, 65, 65), "float32", [], "ragged_transpose"), ((64, 33, 17), "float32", [], "ragged_transpose")]
+
+
+@pytest.mark.parametrize("shape,dtype,ops,want", TRANSPOSES, ids=["%s %s %d" % (s, d, len(o)) for s, d, o, _ in TRANSPOSES])
+def test_planes_that_fill_little_of_a_tile(shape, dtype, ops, want):
+    plan = EN.encode(list(shape), dtype, ops + [EN.Transpose((0, 2, 1))])
+    assert _kernels(plan.blob) == [want]
+
+
+def test_small_planes_under_swapped_outer_axes():
+    for dtype, ops in (("float32", []), ("float32", [F16]), ("int8", [])):
+        plan = EN.encode([64, 64, 8, 8, 8], dtype, [EN.Transpose((0, 4, 2, 1, 3))] + ops)
+        assert _kernels(plan.blob) == ["element"]
 
 
 def test_kernels_of_the_workloads():

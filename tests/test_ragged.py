@@ -52,7 +52,10 @@ TRANSPOSES = [(None, 16, 16), (None, 17, 31), (None, 63, 65), (None, 64, 130), (
               # either side of the smallest c and q that take tiles; the others
               # run element-wise
               (None, 5, 40), (None, 6, 40), (2, 40, 3), (None, 130, 4), (None, 70, 7), (None, 70, 8),
-              (2, 35, 15)]
+              (2, 35, 15),
+              # either side of the fewest elements that a tile may hold, with
+              # the narrowest tiles along c and along q
+              (None, 6, 640), (None, 640, 6), (3, 16, 24), (3, 16, 23), (None, 64, 8), (2, 9, 57)]
 
 
 def transpose_cases(case):
