@@ -322,27 +322,38 @@ bool row_family(int family) {
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Bytes above which a launch's lines do not stay in the 256 MB Infinity Cache
-// until the next launch on other buffers: its rows then come from HBM.
+// Bytes above which little of a launch is still in the 256 MB Infinity Cache
+// when its buffers come round again.
 constexpr int64_t kColdBytes = int64_t{96} << 20;
 
 // Tile widths, order and cache policy of a ragged transpose launch that moves
-// `bytes`. A row that starts inside a line shares it with the next tile.
+// `bytes` and is c_ext wide along c. A row that starts inside a line shares it
+// with the next tile. Figures are over buffers of three calls in turn, which
+// small launches find in the Infinity Cache in part; a second one is over
+// twelve, which none do.
 //   Destination rows that start on 64-byte boundaries: streaming stores of
 //   64 x 64 tiles (int8 [4096,11007] -> f16 24.5 us against 34.8 cached).
 //   Others are written in part by two tiles, which streaming would send to
 //   memory as two partial writes (f32 [16,1001,770] -> f16 16.5 against 13.0
-//   us cached). Cold launches take large tiles, which have fewer such lines,
-//   and streaming loads (f32 [32,2047,513] -> f16, 202 MB, 39.9 us against
-//   49.3 us with 64 x 64 tiles and cached loads); launches that fit the
-//   Infinity Cache take 64 x 64 tiles, of which more run at once (int8
-//   [1027,4099] -> f32, 21 MB, 8.6 against 14.2 us) with cached loads (f32
-//   [16,1001,770] -> f16 13.0 against 15.6 us streaming).
+//   us cached). Large launches (kColdBytes) of planes wider than one 64 x 64
+//   tile along c take large tiles, which have fewer such lines, and streaming
+//   loads (f32 [32,2047,513] -> f16, 202 MB, 38.8 and 46.5 us, small tiles
+//   with cached loads 47.4 and 48.4). Narrower planes would leave half of a
+//   large tile empty (f32 [32768,24,40] 89.0 us, small 51.1; f32 -> f16
+//   [8192,16,128] 44.6, small 23.0). Smaller launches take 64 x 64 tiles, of
+//   which more run at once (int8 [1027,4099] -> f32, 21 MB, 8.6 against 14.2
+//   us; [3637,7047] -> f16, 77 MB, 14.9 and 23.8, large 20.9 and 22.4).
+//   Streaming loads, where rows share lines: large launches only (f32
+//   [16,1001,770] -> f16 13.0 against 15.6 us; f16 [8,4001,1001] 27.8 and
+//   32.0 with large tiles, cached 30.6 and 30.9). Launches whose lines are all
+//   their own keep cached loads at any size: f32 [64,262000] 22.9 and 26.8 us,
+//   streaming 25.5 and 25.6; [16,1040,784] -> f16 12.8 and 18.3, streaming
+//   15.0 and 18.8.
 // Each XCD takes a contiguous run of tiles (74 MB activation above: 18.6 ->
 // 13.0 us), so tiles that share a line meet in one L2, except where no line
 // is shared: words whose rows are all aligned (f32 [262000,64] 22.9 -> 21.0
 // us without).
-void ragged_policy(KArgs &a, int64_t bytes) {
+void ragged_policy(KArgs &a, int64_t bytes, int64_t c_ext) {
   auto aligned = [&](int64_t base, int64_t stride, int64_t batch, int w) {
     return (base * w) % 64 == 0 && (stride * w) % 64 == 0 && (batch * w) % 64 == 0;
   };
@@ -352,7 +363,7 @@ void ragged_policy(KArgs &a, int64_t bytes) {
     dst = dst && aligned(a.dbase, a.t_dsq, a.lv[j].ds, a.wout);
   }
   const bool cold = bytes >= kColdBytes, xcd = a.win == 1 || !src || !dst;
-  const bool large = !dst && cold;
+  const bool large = !dst && cold && c_ext > kRaggedTile;
   a.t_wq = static_cast<uint16_t>(large ? ragged_large_q(a.win) : kRaggedTile);
   a.t_wc = static_cast<uint16_t>(large ? kRaggedLargeC : kRaggedTile);
   a.t_flags = (xcd ? kTileXcd : 0u) | (cold && xcd ? kTileNtLoad : 0u) | (dst ? kTileNtStore : 0u);
@@ -1200,7 +1211,7 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
     batch(dp.qa, dp.ca);
     a.t_ssc = a.ss[dp.ca];
     a.t_dsq = a.ds[dp.qa];
-    ragged_policy(a, box_elements(b, r) * (a.win + a.wout));
+    ragged_policy(a, box_elements(b, r) * (a.win + a.wout), b.ext[dp.ca]);
     const int64_t nq = ceil_div(b.ext[dp.qa], a.t_wq), nc = ceil_div(b.ext[dp.ca], a.t_wc);
     work = box_elements(b, r) / (b.ext[dp.qa] * b.ext[dp.ca]) * nq * nc;
     const int64_t g = std::min<int64_t>(kTileGroup, nq), full = nq / g * g;

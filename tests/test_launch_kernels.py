@@ -119,3 +119,17 @@ def test_refusals():
     assert N.lib().relx_launch_kernels(b._h, 0, out, 4, ctypes.byref(err)) != 0
     assert N.lib().relx_launch_kernels(b._h, 0, None, 4, ctypes.byref(err)) != 0
     assert N.lib().relx_launch_kernels(None, 0, out, 4, ctypes.byref(err)) != 0
+
+
+# Launches of 96 MiB and more whose result rows share lines: tiles 128 wide
+# where the planes are wider than a 64 x 64 tile along c
+LARGE = [((32768, 24, 40), "float32", [], "ragged_transpose"), ((8192, 63, 65), "float32", [], "ragged_transpose"),
+         ((8192, 65, 65), "float32", [], "ragged_transpose_large"), ((32, 2047, 513), "float32", [F16], "ragged_transpose_large"),
+         ((32, 2048, 513), "float32", [F16], "ragged_transpose"), ((2, 2047, 513), "float32", [F16], "ragged_transpose"),
+         ((1, 8001, 8001), "int8", [], "ragged_transpose_large"), ((500000, 20, 60), "int8", [], "ragged_transpose")]
+
+
+@pytest.mark.parametrize("shape,dtype,ops,want", LARGE, ids=["%s %s" % (s, d) for s, d, _, _ in LARGE])
+def test_large_tiles_need_wide_planes(shape, dtype, ops, want):
+    plan = EN.encode(list(shape), dtype, ops + [EN.Transpose((0, 2, 1))])
+    assert _kernels(plan.blob) == [want]
