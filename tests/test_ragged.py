@@ -309,3 +309,63 @@ def test_a_bound_plan_keeps_no_block_of_a_closed_context():
     with P.Context(0) as first, P.Context(0) as second:
         for ctx in (first, second, first, second):
             run(ctx)
+
+
+# Transposes just above the size from which unaligned result rows take large
+# tiles (other kernel bodies with other LDS pitches, streaming loads), both
+# edges cut: one per source width and chain, parameters along either axis.
+LARGE = [((1, 7103, 7107), "int8", None, None), ((1, 5801, 5803), "int8", 0, "float16"),
+         ((1, 5801, 5803), "int8", 1, "float16"), ((1, 4493, 4493), "int8", 1, "float32"),
+         ((1, 4493, 4493), "int8", 0, "float32"), ((1, 5021, 5023), "float16", None, None),
+         ((1, 3551, 3549), "float32", None, None), ((3, 2369, 2371), "float32", None, "float16"),
+         ((3, 2369, 2371), "float32", None, "bfloat16")]
+
+
+def _large_plan(shape, dtype, axis, out, rng):
+    ops = []
+    if axis is not None:
+        n = shape[1 + axis]
+        ops = [EN.Dequantize(_scale(n, rng), zero_point=_zp(n, rng), axis=1 + axis)]
+    if out in ("float16", "bfloat16"):
+        ops.append(EN.Cast(out))
+    return EN.encode(list(shape), dtype, ops + [EN.Transpose((0, 2, 1))]), ops
+
+
+@pytest.mark.parametrize("case", LARGE, ids=[str(c) for c in LARGE])
+def test_large_tile_launches_verify(case):
+    plan, _ = _large_plan(*case, np.random.default_rng(1))
+    b = P.Bound(P.Plan(plan.blob), {}, {})
+    assert P.launch_kernels(b) == ["ragged_transpose_large"]
+    assert P.verify_launches(b, 0, 1 << 30) >= 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", LARGE, ids=[str(c) for c in LARGE])
+def test_large_tiles_on_the_gpu(case):
+    """Bit for bit against torch: the moves are moves, (x - zero point) * scale
+    and the narrowing round once each in both."""
+    torch = pytest.importorskip("torch")
+    shape, dtype, axis, out = case
+    plan, ops = _large_plan(*case, np.random.default_rng(1))
+    b = P.Bound(P.Plan(plan.blob), {}, {})
+    g = torch.Generator(device="cuda").manual_seed(3)
+    if dtype == "int8":
+        x = torch.randint(-128, 128, shape, dtype=torch.int8, device="cuda", generator=g)
+    else:
+        x = torch.randn(shape, dtype=getattr(torch, dtype), device="cuda", generator=g)
+    want = x
+    if axis is not None:
+        view = [1, 1, 1]
+        view[1 + axis] = -1
+        sc, zp = (torch.tensor(p.values, dtype=t, device="cuda").view(view)
+                  for p, t in ((ops[0].scale, torch.float32), (ops[0].zero_point, torch.int32)))
+        want = (x.to(torch.int32) - zp).float() * sc
+    if out in ("float16", "bfloat16"):
+        want = want.to(getattr(torch, out))
+    want = want.transpose(1, 2).contiguous().view(torch.uint8).view(-1)
+    buf = torch.full((want.numel() + 2 * GUARD,), 0xA5, dtype=torch.uint8, device="cuda")
+    with P.Context(0) as ctx:
+        ctx.relayout_device(b, x.data_ptr(), buf.data_ptr() + GUARD, stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+    assert torch.equal(buf[GUARD:-GUARD], want)
+    assert bool((buf[:GUARD] == 0xA5).all()) and bool((buf[-GUARD:] == 0xA5).all())
