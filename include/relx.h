@@ -513,8 +513,9 @@ int relx_verify_launches(const relx_bound *bound, int wire_boundary, int64_t chu
 /* Names of the kernels that relx_relayout_device's launches of this bound
  * plan run with the wire at `wire_boundary` and 16-byte aligned buffers (an
  * indexed plan: relx_index_select_device's), each once, separated by commas:
- * "stream", "flat", "rows", "transpose", "ragged_transpose",
- * "ragged_transpose_large" (tiles 128 wide), "interleave",
+ * "stream", "flat", "rows", "transpose", "transpose_keep" (loads through the
+ * Infinity Cache), "ragged_transpose", "ragged_transpose_large" (tiles 128
+ * wide), "interleave",
  * "ragged_interleave", "permute_shift" and "permute_div" (the direct body,
  * with shifts or divisions), "permute" (the general one), "gather",
  * "gather_cut", "element" and "generic" (one element at a time, in 32 and in

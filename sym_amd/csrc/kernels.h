@@ -854,13 +854,20 @@ __global__ __launch_bounds__(kBlock) void k_transpose(KArgs a) {
                  RELX_NT_STORE(kFamTranspose, WIN, WOUT, 1)>(a);
 }
 
-// Narrowing transposes whose source fits the Infinity Cache beside the result
-// (kTileKeep): cached loads and streaming stores, so that the source stays
-// there rather than the result. f32 [16,1024,768] -> bf16 transposed 14.8 ->
-// 12.4 us where the source is read again while it is there and 15.7 -> 15.6
-// from HBM (buffers of 3 and of 12 calls in turn), [8,2048,1024] -> f16 19.1
-// -> 16.6 and 20.1 -> 19.5; a source of 211 MB, which does not fit, 52.4 ->
-// 55.1.
+// Transposes from four to two bytes of a source of at most 64 MiB (kTileKeep):
+// cached loads and streaming stores, so that the source stays in the Infinity
+// Cache rather than the result. Each figure: buffers of 1, 3, 6 and 12 calls
+// in turn, the other policy before the arrow. The source pays where it is read
+// again while it is there, and costs little where neither side is:
+//   f32 [16,1024,768] -> f16 (50 MB) 14.2 15.0 15.1 15.8 -> 12.3 12.3 15.1 15.5;
+//   f32 [8,2048,1024] -> f16 (67 MB) 19.1 19.1 19.2 20.2 -> 16.6 16.6 19.5 19.5;
+//   f32 [8,1024,1024] -> f16 (34 MB) 9.6 10.4 10.4 10.4 -> 6.6 9.1 9.1 11.1.
+// Larger sources leave the cache while the results of as many calls would
+// stay: f32 [1,4096,8192] -> f16 (134 MB) 35.4 35.4 39.6 39.5 -> 30.7 39.1
+// 39.2 39.2, [28,1024,1024] (117 MB) 30.3 30.4 33.1 32.9 -> 28.6 32.1 32.7
+// 32.8. So do one-byte results, a quarter or half of their source, at any
+// size: f32 [1,4096,4096] -> int8 15.3 16.1 16.1 16.1 -> 14.6 14.6 18.5 18.5,
+// f16 -> int8 11.5 11.8 11.8 11.9 -> 8.2 11.0 11.0 14.2.
 template <int WIN, int WOUT, int CH>
 __global__ __launch_bounds__(kBlock) void k_transpose_keep(KArgs a) {
   transpose_body<WIN, WOUT, CH, kTile, false, true>(a);
@@ -1544,7 +1551,7 @@ hipError_t transpose_launch(const KArgs &a, hipStream_t s) {
     else
       return hipErrorInvalidValue;
   } else if (a.t_flags & kTileKeep) {
-    if constexpr (WIN > WOUT)
+    if constexpr (keeps_source(WIN, WOUT))
       hipLaunchKernelGGL((k_transpose_keep<WIN, WOUT, CH>), grid, block, 0, s, a);
     else
       return hipErrorInvalidValue;

@@ -1195,7 +1195,7 @@ KArgs launch_args(const DeviceProgram &dp, const Box &b, int family) {
       a.t_nc = make_div(nc);
       a.t_full = static_cast<uint32_t>(full);
       a.t_flags = (bytes && !wide ? kTileXcd : 0u) | (wide ? kTileSkew : 0u);
-      if (a.win > a.wout && box_elements(b, r) * a.win <= kKeepBytes)
+      if (keeps_source(a.win, a.wout) && box_elements(b, r) * a.win <= kKeepBytes)
         a.t_flags |= kTileKeep;
       a.t_choff = 0;
       if (a.t_wc == 128 && row_channel(a, b, dp.qa, dp.ca)) {
@@ -1490,7 +1490,7 @@ void verify_launch(const DeviceProgram &dp_in, const KArgs &a, int64_t wire_lo, 
     const int64_t TQ = a.t_wq, TC = a.t_wc;
     if (!(TQ == 64 || (TQ == 128 && win == 1)) || !(TC == 64 || (TC == 128 && TQ == 128)) ||
         a.t_nc.d != a.t_group.d / a.t_g.d || (a.t_flags & ~(kTileXcd | kTileSkew | kTileRowChannel | kTileZeroPoint0 | kTileKeep)) ||
-        ((a.t_flags & kTileKeep) && win <= wout) ||
+        ((a.t_flags & kTileKeep) && !keeps_source(win, wout)) ||
         ((a.t_flags & kTileSkew) && (a.t_flags & kTileXcd)) || (TC == 128 && (a.t_flags & kTileXcd)) ||
         ((a.t_flags & kTileRowChannel) && TC != 128))
       bad_launch(dp, "tile geometry disagrees with the kernel");
@@ -1816,7 +1816,7 @@ const char *launch_kernel(const KArgs &a) {
   case kFamRows:
     return "rows";
   case kFamTranspose:
-    return "transpose";
+    return (a.t_flags & kTileKeep) ? "transpose_keep" : "transpose";
   case kFamRaggedTranspose:
     return a.t_wc == kRaggedLargeC ? "ragged_transpose_large" : "ragged_transpose";
   case kFamInterleave:

@@ -162,10 +162,11 @@ constexpr uint32_t kTileRowChannel = 4;
 // dequantization), so the kernel leaves the subtraction out.
 constexpr uint32_t kTileZeroPoint0 = 8;
 
-// A narrowing transpose whose source is at most kKeepBytes: half the 256 MB
-// Infinity Cache.
+// A transpose from four to two bytes whose source is at most kKeepBytes, a
+// quarter of the 256 MB Infinity Cache (k_transpose_keep).
 constexpr uint32_t kTileKeep = 64;
-constexpr int64_t kKeepBytes = int64_t{128} << 20;
+constexpr int64_t kKeepBytes = int64_t{64} << 20;
+constexpr bool keeps_source(int win, int wout) { return win == 4 && wout == 2; }
 // Ragged transposes: streaming loads, streaming stores.
 constexpr uint32_t kTileNtLoad = 16;
 constexpr uint32_t kTileNtStore = 32;

@@ -133,3 +133,18 @@ LARGE = [((32768, 24, 40), "float32", [], "ragged_transpose"), ((8192, 63, 65), 
 def test_large_tiles_need_wide_planes(shape, dtype, ops, want):
     plan = EN.encode(list(shape), dtype, ops + [EN.Transpose((0, 2, 1))])
     assert _kernels(plan.blob) == [want]
+
+
+# Whole-tile transposes that keep their source in the Infinity Cache: from
+# four to two bytes, sources of at most 64 MiB
+KEEP = [((16, 1024, 768), "float32", [F16], True), ((16, 1024, 1024), "float32", [EN.Cast("bfloat16")], True),
+        ((16, 1024, 1088), "float32", [F16], False), ((2, 4096, 4096), "float32", [F16], False),
+        ((16, 1024, 768), "float32", [EN.Quantize(EN.InlineParam((0.03125,)))], False),
+        ((16, 1024, 768), "float16", [EN.Cast("float32", "exact"), EN.Quantize(EN.InlineParam((0.03125,)))], False),
+        ((16, 1024, 768), "float32", [], False), ((16, 1024, 768), "float16", [EN.Cast("float32", "exact")], False)]
+
+
+@pytest.mark.parametrize("shape,dtype,ops,keep", KEEP, ids=["%s %s %d" % (s, d, i) for i, (s, d, _, _) in enumerate(KEEP)])
+def test_transposes_that_keep_their_source(shape, dtype, ops, keep):
+    plan = EN.encode(list(shape), dtype, ops + [EN.Transpose((0, 2, 1))])
+    assert _kernels(plan.blob) == ["transpose_keep" if keep else "transpose"]
