@@ -516,9 +516,9 @@ int relx_verify_launches(const relx_bound *bound, int wire_boundary, int64_t chu
  * "stream", "flat", "rows", "transpose", "transpose_keep" (loads through the
  * Infinity Cache), "ragged_transpose", "ragged_transpose_large" (tiles 128
  * wide), "interleave",
- * "ragged_interleave", "permute_shift" and "permute_div" (the direct body,
- * with shifts or divisions), "permute" (the general one), "gather",
- * "gather_cut", "element" and "generic" (one element at a time, in 32 and in
+ * "ragged_interleave", "permute_shift GxT" and "permute_div GxT" (the direct body,
+ * with shifts or divisions, in blocks of G channels by T rows), "permute GxT"
+ * (the general one), "gather", "gather_cut", "element" and "generic" (one element at a time, in 32 and in
  * 64 bits: the slow ones); an empty text when nothing is launched. Buffers
  * that are not 16-byte aligned run the stream, flat, transpose, interleave and
  * permute launches element-wise. No counterpart in the reference. */

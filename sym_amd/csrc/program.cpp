@@ -411,19 +411,30 @@ bool direct_chain(const Bound &b, const Prepared &p, uint32_t k, int chain_code,
 }
 
 // Channels G (a divisor of C, at most RELX_PERMUTE_GROUP_BYTES of a source
-// row) and rows T of a direct permute's block: the pair whose blocks keep the
+// row) and rows T of a direct permute's block whose power-of-two pair (G, T)
+// holds fewer than 256 vectors of 16 bytes: the pair whose blocks keep the
 // most of their 256 lanes busy, the cut last m-tile counted, over at most
 // three vectors per lane; among equals the longer row part. f16 -> int8 on the
-// MI355X, general kernel and power-of-two rule -> here: [61,184,40,128] 57.3 ->
-// 30.0 us (10 channels of one row, 160 vectors -> 8 of two, 256), [50,150,32,96]
-// 23.1 -> 14.4 us (192 -> 768), [33,999,8,128] 23.5 -> 17.7 us (odd m: 128 ->
-// 768).
+// MI355X, general kernel and power-of-two rule -> here: [8,1024,40,128] 42.5 ->
+// 21.7 us (10 channels of one row, 160 vectors -> 8 of two, 256),
+// [16,1024,32,96] 45.5 -> 26.9 us (192 -> 768), [33,999,8,128] 35.9 -> 18.0 us
+// (odd m: 128 -> 256).
+// Pairs that fill three quarters of the lanes and store runs of 192 bytes or
+// more only widen G: more rows make a block of several rounds, whose loads
+// and stores alternate (f32 [16,1024,32,96], 8 channels: one row 65.1 us, four
+// 71.9; f32 -> f16 54.0 and 54.2, 384-byte runs; runs of 96 bytes above gain).
+// So do blocks of 256 vectors and more, which keep their pair (f32
+// [8,1024,7,256], 7 channels of one row, 448 vectors, 20.4 us, four rows of one
+// 22.5; f16 [128,196,12,64] 14.5 and 14.6, int8 -> f16 [8,1024,24,128] 14.2 and
+// 15.8).
 void permute_block(int64_t C, int64_t M, int64_t E, int win, int wout, int64_t &G, int64_t &T) {
+  const bool rows = T * G * E * win / 16 < 192 || T * E * wout < 192;
+  const int64_t t_lo = rows ? 1 : T, t_hi = rows ? std::min<int64_t>(8, M) : T;
   double best = 0.0;
   for (int64_t g = C; g >= 1; --g) {
     if (C % g || (g * E * win > RELX_PERMUTE_GROUP_BYTES && g > 1))
       continue;
-    for (int64_t t = 1; t <= std::min<int64_t>(8, M); ++t) {
+    for (int64_t t = t_lo; t <= t_hi; ++t) {
       const int64_t n = t * g * E * win / 16;
       if (t * g * E * wout > 32768 || (n > 3 * 256 && t > 1))
         continue;
@@ -649,10 +660,9 @@ std::unique_ptr<DeviceProgram> build_program(const Bound &b, const Prepared &p, 
         T *= 2;
       ok = T * G * E * wout <= 32768;
     }
-    // blocks that leave lanes idle (their vectors are not a multiple of the
-    // 256 lanes) take another G and T where the launches run the direct
-    // kernel, whose last m-tile may be cut
-    if (ok && (T * G * E / VI) % 256 != 0 && c <= 1 && direct_chain(b, p, k, chain_code, M * E, C))
+    // blocks of fewer vectors than lanes take another G and T where the
+    // launches run the direct kernel, whose last m-tile may be cut
+    if (ok && T * G * E / VI < 256 && c <= 1 && direct_chain(b, p, k, chain_code, M * E, C))
       permute_block(C, M, E, win, wout, G, T);
     if (ok && channels_ok(VI)) {
       family = kFamPermute;
@@ -1078,11 +1088,20 @@ int permute_direct(KArgs &a, int64_t C, int64_t M, int64_t E) {
   const int body = pow2(a.p_ge.d) && pow2(a.p_e.d) && pow2(a.p_run.d) && a.p_m % a.p_t == 0
                        ? kPermuteShift
                        : kPermuteDiv;
+  const int k = chain_param_stage(a.chain_code);
+  // Blocks of several vectors per lane without parameters, from four-byte
+  // sources: the direct kernel saves no channel there, and the general one has
+  // four vectors of a lane in flight for its two (f32 -> f16 [8,512,3,1024]
+  // 13.6 us, direct 14.5; f32 [16,1024,5,128] 14.8 and 15.3, [8,1024,7,256]
+  // 20.6 and 20.4; f16 [64,512,6,32] 6.4 and 5.5, int8 [8,1024,16,80] 6.4 and
+  // 5.0).
+  if (body == kPermuteDiv && a.win == 4 && k < 0 && a.p_m % a.p_t == 0 &&
+      a.p_t * a.p_ge.d * 4 / 16 > 256)
+    return kPermuteGeneral;
   // the direct kernel takes a batch entry's offsets from the innermost level
   for (int j = 0; j + 1 < kBatchLevels; ++j)
     if (a.lv[j].div.d != 1 || a.lv[j].vcnt != 1)
       return kPermuteGeneral;
-  const int k = chain_param_stage(a.chain_code);
   if (k < 0)
     return body;
   const DevStage &s = a.chain.st[k];
@@ -1807,7 +1826,7 @@ int64_t launch_program(const DeviceProgram &dp, int64_t v0, int64_t v1, bool fir
                     part ? v0 * dp.chunk_stride : 0, part ? v1 * dp.chunk_stride : -1);
 }
 
-const char *launch_kernel(const KArgs &a) {
+std::string launch_kernel(const KArgs &a) {
   switch (a.family) {
   case kFamStream:
     return "stream";
@@ -1824,7 +1843,10 @@ const char *launch_kernel(const KArgs &a) {
   case kFamRaggedInterleave:
     return "ragged_interleave";
   case kFamPermute:
-    return a.p_direct == kPermuteShift ? "permute_shift" : a.p_direct == kPermuteDiv ? "permute_div" : "permute";
+    return std::string(a.p_direct == kPermuteShift ? "permute_shift "
+                       : a.p_direct == kPermuteDiv ? "permute_div "
+                                                   : "permute ") +
+           std::to_string(a.p_g) + "x" + std::to_string(a.p_t);
   case kFamElement:
     return "element";
   default:

@@ -91,7 +91,7 @@ std::vector<KArgs> axis_launches(const DeviceProgram &dp, int axis, int64_t plo,
 std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed, int axis,
                                    int64_t plo, int64_t phi, bool resident = false);
 // The kernel that a laid out launch runs (relx_launch_kernels).
-const char *launch_kernel(const KArgs &a);
+std::string launch_kernel(const KArgs &a);
 // Coordinates a box along axis i must keep together (0: never split).
 int64_t axis_align(const DeviceProgram &dp, int i);
 // Launch boxes (verified first when RELX_VERIFY_LAUNCHES is set, their

@@ -42,8 +42,8 @@ def test_kernels_of_the_ragged_groups(kind):
         mine = set()
         for name, blob, _ in make(case):
             got = _kernels(blob)
-            assert len(got) == 1 and got[0] in GROUP_KERNELS[kind], (name, got)
-            mine.update(got)
+            assert len(got) == 1 and got[0].split()[0] in GROUP_KERNELS[kind], (name, got)
+            mine.add(got[0].split()[0])
         if kind == "rows":
             assert "rows" in mine, case
         if kind == "transpose" and case[1] * case[2] >= 500 and min(case[1:]) >= 9:
@@ -60,11 +60,36 @@ def test_kernels_of_the_permutes(case):
     name, blob, _, direct = case
     want = "permute_shift" if direct else "permute" if " per D" in name or " per S" in name or "batch" in name \
         else "permute_div"
-    assert _kernels(blob) == [want]
+    assert [k.split()[0] for k in _kernels(blob)] == [want]
 
 
 def test_random_permutes_take_every_body():
-    assert {_kernels(blob)[0] for _, blob, _ in PC.random_cases(200)} == {"permute_shift", "permute_div", "permute"}
+    assert {_kernels(blob)[0].split()[0] for _, blob, _ in PC.random_cases(200)} == \
+        {"permute_shift", "permute_div", "permute"}
+
+
+def _head_quant(heads):
+    return [EN.Cast("float32", "exact"),
+            EN.Quantize(EN.InlineParam(tuple(0.01 + 0.001 * i for i in range(heads)), "float32", 1), axis=1)]
+
+
+# [B, S, H, D] -> [B, H, S, D]: the body and the block (heads by rows of S).
+# Blocks of 256 vectors and more, and blocks that fill three quarters of the
+# lanes and store whole lines, keep their power-of-two pair of H and S.
+PERMUTES = [((8, 1024, 7, 256), "float32", None, "permute 7x1"), ((8, 1024, 7, 256), "float16", None, "permute_div 7x2"),
+            ((16, 1024, 32, 96), "float32", None, "permute_div 8x1"), ((16, 1024, 32, 96), "float16", None, "permute_div 16x1"),
+            ((16, 1024, 32, 96), "float16", _head_quant(32), "permute_div 16x4"),
+            ((128, 196, 12, 64), "float32", None, "permute 12x2"), ((128, 196, 12, 64), "float32", [EN.Cast("float16")], "permute 12x2"),
+            ((128, 197, 12, 64), "float32", None, "permute_div 12x1"), ((128, 197, 12, 64), "float16", None, "permute_div 12x8"),
+            ((8, 1024, 40, 128), "float32", None, "permute_shift 8x1"), ((8, 1024, 40, 128), "float16", _head_quant(40), "permute_shift 8x2"),
+            ((8, 512, 3, 1024), "float32", [EN.Cast("float16")], "permute 3x1"), ((8, 1024, 16, 80), "int8", None, "permute_div 16x4"),
+            ((33, 999, 8, 128), "float16", _head_quant(8), "permute_div 8x2"), ((32, 1000, 8, 128), "float16", None, "permute_shift 8x4"),
+            ((8, 4096, 32, 128), "float16", _head_quant(32), "permute_shift 16x1")]
+
+
+@pytest.mark.parametrize("shape,dtype,ops,want", PERMUTES, ids=["%s %s %s" % (s, d, w) for s, d, _, w in PERMUTES])
+def test_permute_blocks(shape, dtype, ops, want):
+    assert _kernels(EN.encode(list(shape), dtype, [EN.Transpose((0, 2, 1, 3))] + (ops or [])).blob) == [want]
 
 
 DEQ = EN.Dequantize(EN.InlineParam((0.03125,)))
@@ -99,7 +124,8 @@ def test_kernels_of_the_workloads():
     assert _kernels(W.c3_plan().blob, {"s0": 4096, "s1": 11008},
                     W.param("scale", np.ones(11008, np.float32))) == ["transpose"]
     assert _kernels(W.c4_plan().blob, {"s0": 512, "s1": 256}, W.param("scale", np.ones(512, np.float32))) == ["stream"]
-    assert _kernels(W.c5_plan().blob, {"B": 2, "S": 64}, W.param("scale", np.ones(32, np.float32))) == ["permute_shift"]
+    assert _kernels(W.c5_plan().blob, {"B": 2, "S": 64}, W.param("scale", np.ones(32, np.float32))) == \
+        ["permute_shift 16x1"]
 
 
 def test_kernels_of_a_row_gather():
