@@ -326,6 +326,14 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // when its buffers come round again.
 constexpr int64_t kColdBytes = int64_t{96} << 20;
 
+// A stage takes another parameter entry for each element of a vector.
+bool channel_per_element(const KArgs &a) {
+  for (int i = 0; i < a.chain.n; ++i)
+    if (a.chain.st[i].vec == 1)
+      return true;
+  return false;
+}
+
 // Tile widths, order and cache policy of a ragged transpose launch that moves
 // `bytes` and is c_ext wide along c. A row that starts inside a line shares it
 // with the next tile. Figures are over buffers of three calls in turn, which
@@ -340,7 +348,9 @@ constexpr int64_t kColdBytes = int64_t{96} << 20;
 //   loads (f32 [32,2047,513] -> f16, 202 MB, 38.8 and 46.5 us, small tiles
 //   with cached loads 47.4 and 48.4). Narrower planes would leave half of a
 //   large tile empty (f32 [32768,24,40] 89.0 us, small 51.1; f32 -> f16
-//   [8192,16,128] 44.6, small 23.0). Smaller launches take 64 x 64 tiles, of
+//   [8192,16,128] 44.6, small 23.0), and a channel per element of a row, whose
+//   entries every vector loads, leaves them behind at any width (int8 -> f16
+//   [8208,8192] scaled along c 144, small 101). Smaller launches take 64 x 64 tiles, of
 //   which more run at once (int8 [1027,4099] -> f32, 21 MB, 8.6 against 14.2
 //   us; [3637,7047] -> f16, 77 MB, 14.9 and 23.8, large 20.9 and 22.4).
 //   Streaming loads, where rows share lines: large launches only (f32
@@ -363,7 +373,7 @@ void ragged_policy(KArgs &a, int64_t bytes, int64_t c_ext) {
     dst = dst && aligned(a.dbase, a.t_dsq, a.lv[j].ds, a.wout);
   }
   const bool cold = bytes >= kColdBytes, xcd = a.win == 1 || !src || !dst;
-  const bool large = !dst && cold && c_ext > kRaggedTile;
+  const bool large = !dst && cold && c_ext > kRaggedTile && !channel_per_element(a);
   a.t_wq = static_cast<uint16_t>(large ? ragged_large_q(a.win) : kRaggedTile);
   a.t_wc = static_cast<uint16_t>(large ? kRaggedLargeC : kRaggedTile);
   a.t_flags = (xcd ? kTileXcd : 0u) | (cold && xcd ? kTileNtLoad : 0u) | (dst ? kTileNtStore : 0u);
@@ -373,7 +383,8 @@ void ragged_policy(KArgs &a, int64_t bytes, int64_t c_ext) {
 // cut run as one ragged launch, and a device-resident call's whatever their
 // size (f32 [128,96] -> f16 transposed 11.0 us a pass as tiles and a strip,
 // 7.0 as one launch; [72,200], with two strips, 14.7 and 7.0). A smaller box
-// of a transfer keeps its whole tiles and strips.
+// of a transfer keeps its whole tiles and strips, and so do the boxes of
+// tiles_and_strips.
 constexpr int64_t kRaggedWholeElements = int64_t{1} << 14;
 
 // The ragged transpose needs one vector of q and takes c extents from here on:
@@ -1022,6 +1033,31 @@ void element_args(const DeviceProgram &dp, const Box &b, KArgs &a) {
   }
 }
 
+// Large aligned transpose boxes (kColdBytes) with cut tiles that keep their
+// whole tiles on the tile kernel and run the strips past them as ragged
+// launches:
+// - a channel per element of rows that start off 64-byte boundaries: such rows
+//   want large tiles, which such chains make slow (ragged_policy). int8 -> f16
+//   [8208,8192] scaled along c 88.9 us, one ragged launch 144 (small tiles
+//   101); f32 -> int8 78.9 and 91.6.
+// - one-byte sources of four-byte results whose source rows lie multiples of 8
+//   KiB apart: a ragged tile reads 64-byte halves of lines that fall on the
+//   same sets, and the other halves are gone when the next tile wants them; the
+//   tile kernel's rows are whole lines. int8 -> f32 [4112,8192] 34.7 us, one
+//   ragged launch 50.6; [8208,8192] 59.7 and 65.8; rows 6 or 12 KiB apart 32.2
+//   and 26.0, 52.9 and 51.2.
+bool tiles_and_strips(const DeviceProgram &dp, const Box &b) {
+  const KArgs &a = dp.base;
+  if (box_elements(b, a.rank) * (a.win + a.wout) < kColdBytes)
+    return false;
+  if (a.win == 1 && a.wout == 4 && a.ss[dp.ca] % 8192 == 0)
+    return true;
+  bool aligned = true;
+  for (int i = 0; i < a.rank; ++i)
+    aligned = aligned && (i == dp.ca || b.ext[i] <= 1 || (a.ds[i] * a.wout) % 64 == 0);
+  return !aligned && channel_per_element(a);
+}
+
 // Arguments of an edge box: the element-wise kernel over the box.
 KArgs edge_args(const DeviceProgram &dp, const Box &b) {
   KArgs a = dp.base;
@@ -1323,8 +1359,8 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
   std::vector<KArgs> out;
   std::vector<Box> edges;
   // A transpose box whose q or c extent is not a multiple of the tile runs
-  // as one ragged launch; a transfer's small one keeps its whole tiles on the
-  // tile kernel and runs the strips past them (the q strip over the whole c
+  // as one ragged launch; a transfer's small one, and those of
+  // tiles_and_strips, keep their whole tiles on the tile kernel and run the strips past them (the q strip over the whole c
   // range, the c strip beside the whole q tiles) as ragged launches.
   int family = dp.family;
   if (family == kFamStream && a.rank == 1 && b.ext[0] % a.vec != 0)
@@ -1339,7 +1375,7 @@ std::vector<KArgs> prefix_launches(const DeviceProgram &dp, const int64_t *fixed
   if (family == kFamRaggedInterleave && b.ext[a.rank - 2] < a.vec)
     return {edge_args(dp, b)};
   if (family == kFamTranspose && (b.ext[dp.qa] % a.t_wq || b.ext[dp.ca] % a.t_wc)) {
-    if (resident || box_elements(b, a.rank) >= kRaggedWholeElements) {
+    if ((resident || box_elements(b, a.rank) >= kRaggedWholeElements) && !tiles_and_strips(dp, b)) {
       family = kFamRaggedTranspose;
     } else {
       const int q = dp.qa, c = dp.ca;

@@ -174,3 +174,31 @@ KEEP = [((16, 1024, 768), "float32", [F16], True), ((16, 1024, 1024), "float32",
 def test_transposes_that_keep_their_source(shape, dtype, ops, keep):
     plan = EN.encode(list(shape), dtype, ops + [EN.Transpose((0, 2, 1))])
     assert _kernels(plan.blob) == ["transpose_keep" if keep else "transpose"]
+
+
+def _scale(n):
+    return EN.InlineParam(tuple(0.01 + 0.001 * (i % 50) for i in range(n)), "float32", 1)
+
+
+# Large aligned transposes [r, q] whose last tiles are cut: one ragged launch,
+# or whole tiles and ragged strips (a channel per element of unaligned rows;
+# one-byte rows 8 KiB apart to f32)
+CUT = [((4112, 11008), "int8", 0, "float16", ["transpose", "ragged_transpose"]),
+       ((4112, 11008), "int8", 1, "float16", ["ragged_transpose_large"]),
+       ((4128, 11008), "int8", 0, "float16", ["ragged_transpose"]),
+       ((2064, 2064), "int8", 0, "float16", ["ragged_transpose"]),
+       ((8208, 8192), "float32", 0, "int8", ["transpose", "ragged_transpose"]),
+       ((4112, 8192), "int8", 1, "float32", ["transpose", "ragged_transpose"]),
+       ((1040, 8192), "int8", 1, "float32", ["ragged_transpose"]),
+       ((4112, 6144), "int8", 1, "float32", ["ragged_transpose"]),
+       ((4112, 8192), "int8", 1, "float16", ["ragged_transpose_large"]),
+       ((7001, 7003), "int8", 0, "float16", ["ragged_transpose"])]
+
+
+@pytest.mark.parametrize("shape,dtype,axis,out,want", CUT, ids=["%s %s %d %s" % c[:4] for c in CUT])
+def test_cut_tiles_of_large_transposes(shape, dtype, axis, out, want):
+    sc = _scale(shape[axis])
+    ops = [EN.Quantize(sc, axis=axis)] if out == "int8" else [EN.Dequantize(sc, axis=axis)]
+    plan = EN.encode(list(shape), dtype, ops + ([F16] if out == "float16" else []) + [EN.Transpose((1, 0))])
+    assert _kernels(plan.blob) == want
+    assert P.verify_launches(P.Bound(P.Plan(plan.blob), {}, {}), 0, 1 << 30) >= len(want)

@@ -313,12 +313,15 @@ def test_a_bound_plan_keeps_no_block_of_a_closed_context():
 
 # Transposes just above the size from which unaligned result rows take large
 # tiles (other kernel bodies with other LDS pitches, streaming loads), both
-# edges cut: one per source width and chain, parameters along either axis.
+# edges cut: one per source width and chain, parameters along either axis (a
+# channel per element of a row takes small tiles, or with aligned source rows
+# whole tiles and strips, as one-byte rows 8 KiB apart do to f32).
 LARGE = [((1, 7103, 7107), "int8", None, None), ((1, 5801, 5803), "int8", 0, "float16"),
          ((1, 5801, 5803), "int8", 1, "float16"), ((1, 4493, 4493), "int8", 1, "float32"),
          ((1, 4493, 4493), "int8", 0, "float32"), ((1, 5021, 5023), "float16", None, None),
          ((1, 3551, 3549), "float32", None, None), ((3, 2369, 2371), "float32", None, "float16"),
-         ((3, 2369, 2371), "float32", None, "bfloat16")]
+         ((3, 2369, 2371), "float32", None, "bfloat16"), ((1, 4112, 11008), "int8", 0, "float16"),
+         ((1, 4112, 8192), "int8", 1, "float32")]
 
 
 def _large_plan(shape, dtype, axis, out, rng):
@@ -335,7 +338,12 @@ def _large_plan(shape, dtype, axis, out, rng):
 def test_large_tile_launches_verify(case):
     plan, _ = _large_plan(*case, np.random.default_rng(1))
     b = P.Bound(P.Plan(plan.blob), {}, {})
-    assert P.launch_kernels(b) == ["ragged_transpose_large"]
+    shape, dtype, axis, out = case
+    if shape[2] % 16 == 0:
+        want = ["transpose", "ragged_transpose"]
+    else:
+        want = ["ragged_transpose" if axis == 0 else "ragged_transpose_large"]
+    assert P.launch_kernels(b) == want
     assert P.verify_launches(b, 0, 1 << 30) >= 1
 
 
