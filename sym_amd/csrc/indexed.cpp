@@ -160,6 +160,23 @@ void verify_gather(const Bound &b, const GatherPlan &g, const std::vector<Gather
                 g.row_units * (g.op == kGatherCopy ? 1 : static_cast<int64_t>(sw)) != row_in
           : row_in != g.row_items * g.nbi || row_out != g.row_items * g.nbo)
     bad("row length disagrees with the vector shape");
+  // the kernel's items of a cut row: loads inside the table row, stores that
+  // continue one another up to the end of the result row
+  if (cut) {
+    const int64_t V = g.op == kGatherCopy ? g.nbi : g.nbi / static_cast<int64_t>(sw);
+    const int64_t wi = g.nbi / V, wo = g.nbo / V;
+    int64_t stored = 0;
+    for (int64_t j = 0; j < g.row_items; ++j) {
+      const int64_t at = j * V, back = std::max<int64_t>(0, at + V - g.row_units);
+      if (at < back || back >= V || (at - back) * wi + g.nbi > row_in)
+        bad("an item loads outside its table row");
+      if (at * wo != stored)
+        bad("an item does not continue the previous one");
+      stored += (V - back) * wo;
+    }
+    if (stored != row_out)
+      bad("the items of a row do not cover it");
+  }
   if (b.table_rows * row_in > static_cast<int64_t>(table_bytes))
     bad("table rows exceed the table buffer");
   for (int64_t v : b.indices)

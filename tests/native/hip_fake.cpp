@@ -856,7 +856,6 @@ hipError_t gather_launch(const GatherArgs &a, int op, int nbi, int iw, bool nt, 
   (void)nt;
   if (a.work == 0)
     return hipSuccess;
-  (void)nbi;
   const int64_t rows = (static_cast<int64_t>(a.work) + a.row_items - 1) / a.row_items;
   const int64_t row_bytes = a.row_src;
   std::lock_guard<std::mutex> g(g_mu);
@@ -879,14 +878,24 @@ hipError_t gather_launch(const GatherArgs &a, int op, int nbi, int iw, bool nt, 
       {{t + static_cast<uintptr_t>(lo * row_bytes), t + static_cast<uintptr_t>((hi + 1) * row_bytes)},
        {ix, ix + static_cast<uintptr_t>(rows * iw)}},
       {d, d + static_cast<uintptr_t>(rows * a.row_dst)},
-      [k, op, rows, iw] {
-        for (int64_t r = 0; r < rows; ++r) {
+      [k, op, nbi, iw] { // item by item, as the kernels; conversions store zeros
+        const int64_t in_w = op == kGatherCopy ? 1 : op == kGatherF32F16 ? 4 : 2;
+        const int64_t out_w = op == kGatherCopy ? 1 : op == kGatherF32F16 ? 2 : 4;
+        const int64_t V = nbi / in_w; // units of an item
+        for (int64_t i = 0; i < static_cast<int64_t>(k.work); ++i) {
+          const int64_t r = i / k.row_items, at = (i - r * k.row_items) * V;
+          // a cut row's last item is loaded from the row's last bytes
+          const int64_t back = k.row_units && at + V > k.row_units ? at + V - k.row_units : 0;
           const int64_t row = iw == 8 ? reinterpret_cast<const int64_t *>(k.idx)[r]
                                       : reinterpret_cast<const int32_t *>(k.idx)[r];
+          uint8_t item[16];
+          std::memcpy(item, k.table + row * k.row_src + (at - back) * in_w, static_cast<size_t>(nbi));
+          uint8_t *out = k.dst + r * k.row_dst + at * out_w;
+          const size_t n = static_cast<size_t>((V - back) * out_w);
           if (op == kGatherCopy)
-            std::memcpy(k.dst + r * k.row_dst, k.table + row * k.row_src, static_cast<size_t>(k.row_src));
+            std::memcpy(out, item + back, n);
           else
-            std::memset(k.dst + r * k.row_dst, 0, static_cast<size_t>(k.row_dst));
+            std::memset(out, 0, n);
         }
       }));
 }

@@ -133,6 +133,13 @@ def cases(tmp_path_factory):
     iplan = EN.encode_index_select(["N", "D"], "float32", "M", "int64", "float32")
     syms = {"N": 4096, "D": 64, "M": len(idx)}
     c["ix"] = write_case(root, "ix", iplan, table, table[idx].tobytes(), syms, index=(64, idx))
+    # rows of 1001 and of 30 bytes: 16-byte items whose last one is cut
+    for name, dt, d in (("ix_cut", np.int8, 1001), ("ix_short", np.int16, 15)):
+        table = rng.integers(-100, 100, (512, d)).astype(dt)
+        idx = rng.integers(0, 512, 700).astype(np.int64)
+        plan = EN.encode_index_select([512, d], "int8" if dt is np.int8 else "float16", 700, "int64",
+                                      "int8" if dt is np.int8 else "float16")
+        c[name] = write_case(root, name, plan, table, table[idx].tobytes(), {}, index=(64, idx))
     # a (128, 96) f16 transpose: a tile kernel and an edge kernel read the
     # one chunk
     src = np.random.default_rng(255).standard_normal((128, 96)).astype(np.float16)
@@ -305,7 +312,8 @@ def test_device_to_host_and_device_resident(driver, cases):
             lines.append("device %s caller=%s %s" % (cases[name], caller, DELAYS))
     lines.append("d2h %s caller=null %s" % (cases["c1"], DELAYS))
     # an indexed plan's rows gathered from a device-resident table
-    lines += ["device %s caller=%s %s" % (cases["ix"], caller, DELAYS) for caller in ("null", "stream")]
+    lines += ["device %s caller=%s %s" % (cases[name], caller, DELAYS)
+              for name in ("ix", "ix_cut", "ix_short") for caller in ("null", "stream")]
     res = run(driver, lines)
     for r in res:
         ok(r)
