@@ -15,6 +15,7 @@
 // branch -- both on the kernel's critical path.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
 
 namespace relx {
@@ -278,8 +279,9 @@ struct KArgs {
 enum PermuteBody : int32_t { kPermuteGeneral = 0, kPermuteShift = 1, kPermuteDiv = 2 };
 
 // Arguments of a direct permute launch (KArgs::p_direct): only the fields its
-// blocks read, 34 dwords that a block fetches in one round of scalar loads.
-// (Built from KArgs, 2,024 bytes, whose fields the general kernel reads from
+// blocks read, 34 dwords with shifts and 42 with divisions, which a block
+// fetches in one round of scalar loads.
+// (Built from KArgs, 2,072 bytes, whose fields the general kernel reads from
 // its first 656 in three dependent rounds, spilling scalar registers, before
 // its first data load; with blocks of 4-8 KiB of source that start costs C5
 // [8,4096,32,128] 20%.) The
@@ -305,6 +307,8 @@ struct PermArgs {
   uint32_t ge_d, ge_m, e_d, e_m, run_d, run_m; // kPermuteDiv: FastDivs (shifts above)
   uint32_t m;                                  // kPermuteDiv: m of the box
 };
+static_assert(sizeof(KArgs) == 2072 && offsetof(PermArgs, ge_d) == 34 * 4 && sizeof(PermArgs) == 42 * 4,
+              "the sizes named above");
 
 // Row gather of an indexed plan (index_select along axis 0, at most one cast):
 // a launch covers `work` vector items of consecutive selected rows, each row

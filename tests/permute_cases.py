@@ -1,10 +1,11 @@
 """Block-permute plans ([B, S, H, D] -> [B, H, S, D] with value stages) that
-take the direct permute body or keep the general one.
+take each of the three permute bodies.
 
-The direct body (power-of-two H*D, D and store runs; the parameter stage,
-if any, per tensor or per channel along H) indexes with shifts and takes a
-vector's parameters from its own H coordinate. Every other permute derives
-the channel from the dense result offset. Used by the CPU launch checks
+The direct body (the parameter stage, if any, per tensor or per channel along
+H) takes a vector's parameters from its own H coordinate, and indexes with
+shifts where H*D, D and the store runs are powers of two (the `direct` cases)
+and with divisions elsewhere. The general body derives the channel from the
+dense result offset. Used by the CPU launch checks
 (which body each plan gets; every launch verified) and by the GPU parity
 test against the oracle.
 """
@@ -35,7 +36,7 @@ def cases(B=2, S=64):
             x = (rng.standard_normal(shape) * 3).astype(dtype)
         out.append((name, EN.encode(list(shape), dtype, [perm] + ops).blob, x, direct))
 
-    # direct: one case per compile-time chain
+    # direct with shifts: one case per compile-time chain
     add("f16 quant per head", 32, 128, "float16",
         [EN.Cast("float32", "exact"), EN.Quantize(_per(32, rng), axis=1)], True)
     add("f16 quant per tensor", 32, 128, "float16",
@@ -50,13 +51,14 @@ def cases(B=2, S=64):
     add("f32 -> f16", 32, 128, "float32", [EN.Cast("float16")], True)
     add("f16 -> f32", 32, 128, "float16", [EN.Cast("float32", "exact")], True)
     add("f16 layout only", 32, 128, "float16", [], True)
-    # general body: the channel is not H, or a division is not a shift
+    # general body: the channel is not H
     add("f16 quant per D", 32, 128, "float16",
         [EN.Cast("float32", "exact"), EN.Quantize(_per(128, rng), axis=3)], False)
     add("f16 quant per S", 32, 128, "float16",
         [EN.Cast("float32", "exact"), EN.Quantize(_per(S, rng), axis=2)], False)
     add("f16 quant per batch", 32, 128, "float16",
         [EN.Cast("float32", "exact"), EN.Quantize(_per(B, rng), axis=0)], False)
+    # direct with divisions: a division is not a shift
     add("f16 quant per head, 24 heads", 24, 128, "float16",
         [EN.Cast("float32", "exact"), EN.Quantize(_per(24, rng), axis=1)], False)
     add("f16 quant per head, D = 96", 32, 96, "float16",
