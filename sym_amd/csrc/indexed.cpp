@@ -97,27 +97,44 @@ GatherPlan gather_plan(const Bound &b, const void *table, const void *dst) {
   g.row_items = b.row_elements * sw / g.nbi;
   // Rows whose length or buffers allow only narrow whole items move in
   // 16-byte items at any alignment, the last one of each row cut, where that
-  // measured faster (whole narrow items -> cut wide ones, 32-64 Ki rows and
-  // equal bytes of shorter ones):
-  //   copies by 1 or 2 bytes: int8 rows of 1001 bytes 107 -> 29 us, 31 bytes
-  //   67 -> 37;
-  //   copies by 4 bytes, rows of at least 128 bytes: 4004 bytes 78 -> 55, 252
-  //   bytes 38.9 -> 36.5, 124 bytes 43.7 -> 43.8, 60 bytes 48.8 -> 52.7;
-  //   f32 -> f16 by 4 bytes, rows of at least 32: 4004 bytes 73 -> 37, 60
-  //   bytes 46 -> 42, 20 bytes 93.7 -> 99.5.
+  // measured faster over tables of 32 Ki to 1 Mi rows and selections of 64 and
+  // 256 Ki (whole narrow items -> cut wide ones, us; n/m: n rows of m Ki):
+  //   copies by single bytes: 31 bytes 256/1024 13.0 -> 10.2, 1001 bytes
+  //   64/256 106.3 -> 29.0;
+  //   copies by 2 bytes, rows of at least 32: 34 bytes 256/32 8.0 -> 6.7 and
+  //   256/1024 9.8 -> 9.2; 18 bytes 4.9 -> 5.2 and 7.9 -> 7.8;
+  //   copies by 4 bytes, rows of at least 768, or 4000 where the selection has
+  //   more rows than the table and reads them from the caches: 1004 bytes
+  //   64/256 31.0 -> 28.2, 256/256 151.6 -> 110.7, 256/1024 156.1 -> 116.1,
+  //   256/32 89.9 -> 97.0, 4004 bytes 256/32 417 -> 398; 132 bytes 256/1024
+  //   17.9 -> 20.6, 252 bytes 256/256 27.7 -> 31.0, 324 bytes 34.1 -> 38.3,
+  //   644 bytes 64/256 17.4 -> 19.5 (but 256/1024 101.8 -> 77.1);
+  //   f32 -> f16 by 4 bytes, rows of at least 32: 36 bytes 256/32 5.5 -> 5.1,
+  //   124 bytes 256/1024 16.6 -> 15.1, 1004 bytes 64/256 36.4 -> 24.1.
   // Whole items of 8 bytes keep up (f32 rows of 4008 bytes 53.0, cut 55.2),
   // and so do the widening f16 rows (254 bytes 21.8, cut 28.5).
   const int64_t row_bytes = b.row_elements * sw;
-  const int64_t cut_from = g.op == kGatherCopy     ? (g.nbi <= 2 ? 16 : g.nbi == 4 ? 128 : INT64_MAX)
-                           : g.op == kGatherF32F16 ? (g.nbi == 4 ? 32 : INT64_MAX)
-                                                   : INT64_MAX;
+  const int64_t count = static_cast<int64_t>(b.indices.size());
+  int64_t cut_from = INT64_MAX;
+  if (g.op == kGatherCopy && g.nbi <= 4)
+    cut_from = g.nbi == 1 ? 16 : g.nbi == 2 ? 32 : count <= b.table_rows ? 768 : 4000;
+  else if (g.op == kGatherF32F16 && g.nbi == 4)
+    cut_from = 32;
+  bool stream = row_bytes >= 256;
   if (row_bytes >= cut_from && row_bytes < kMaxLaunchWork) {
+    // Neighbouring cut items share lines. Where whole items would be of 4 bytes
+    // and go through the caches, cut ones stream only long rows (f32 -> f16,
+    // 260 bytes 64/256 whole 8.2, cached 7.9, streaming 8.9; 2004 bytes 64/256
+    // 72.6, 42.5, 39.1), and copies only tables larger than their selection
+    // (1004 bytes 256/256 110.7 cached, 118.6 streaming; 64/256 32.1, 28.2).
+    if (g.nbi == 4)
+      stream = row_bytes >= 768 && (g.op != kGatherCopy || count < b.table_rows);
     g.row_units = g.op == kGatherCopy ? row_bytes : b.row_elements;
     g.nbi = 16;
     g.nbo = g.op == kGatherCopy ? 16 : 8;
     g.row_items = (row_bytes + 15) / 16;
   }
-  g.nt = g.nbi >= 8 && row_bytes >= 256;
+  g.nt = g.nbi >= 8 && stream;
   if (g.row_items >= kMaxLaunchWork)
     throw Error("unsupported_layout", "an indexed row spans 2^31 or more vector items");
   return g;

@@ -128,11 +128,32 @@ def test_kernels_of_the_workloads():
         ["permute_shift 16x1"]
 
 
-def test_kernels_of_a_row_gather():
-    for d, want in ((1024, ["gather"]), (1001, ["gather_cut"])):
-        blob = EN.encode_index_select([64, d], "int8", 8, "int64", "int8")
-        idx = np.arange(8, dtype="<i8")
-        assert P.launch_kernels(P.bind_indexed(P.load_indexed_plan(blob), {}, ("int64", [8], idx.tobytes()))) == want
+# (table dtype, result dtype, elements of a row, kernel) on either side of each
+# length from which rows move in cut 16-byte items
+GATHERS = [("int8", "int8", 15, "gather"), ("int8", "int8", 17, "gather_cut"), ("int8", "int8", 30, "gather"),
+           ("int8", "int8", 31, "gather_cut"), ("int8", "int8", 34, "gather_cut"), ("int8", "int8", 764, "gather"),
+           ("int8", "int8", 772, "gather_cut"), ("int8", "int8", 1001, "gather_cut"), ("int8", "int8", 1024, "gather"),
+           ("float16", "float16", 15, "gather"), ("float16", "float16", 17, "gather_cut"),
+           ("float32", "float32", 33, "gather"), ("float32", "float32", 191, "gather"),
+           ("float32", "float32", 193, "gather_cut"), ("float32", "float32", 194, "gather"),
+           ("float32", "float16", 7, "gather"), ("float32", "float16", 9, "gather_cut"),
+           ("float16", "float32", 501, "gather")]
+
+
+def _gather_kernels(rows, d, src, count, dst):
+    blob = EN.encode_index_select([rows, d], src, count, "int64", dst)
+    idx = (np.arange(count) % rows).astype("<i8")
+    return P.launch_kernels(P.bind_indexed(P.load_indexed_plan(blob), {}, ("int64", [count], idx.tobytes())))
+
+
+@pytest.mark.parametrize("src,dst,d,want", GATHERS, ids=["%s-%s %d" % g[:3] for g in GATHERS])
+def test_kernels_of_a_row_gather(src, dst, d, want):
+    assert _gather_kernels(64, d, src, 8, dst) == [want]
+
+
+def test_word_rows_that_a_selection_reads_again_keep_whole_items():
+    for d, count, want in ((251, 64, "gather_cut"), (251, 65, "gather"), (999, 65, "gather"), (1001, 65, "gather_cut")):
+        assert _gather_kernels(64, d, "float32", count, "float32") == [want], (d, count)
 
 
 def test_refusals():

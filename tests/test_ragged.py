@@ -242,8 +242,9 @@ def test_results_on_the_gpu(group):
 # (table dtype, result dtype, row elements): rows of one 16-byte item, of one
 # element more and less than items, and on either side of each length from
 # which rows move in cut items
-GATHERS = [("int8", "int8", (15, 16, 17, 31, 33, 127, 1001)), ("float16", "float16", (7, 8, 9, 17, 63, 501)),
-           ("float32", "float32", (5, 31, 32, 33, 63, 1001)), ("float32", "float16", (7, 8, 9, 11, 33, 1001)),
+GATHERS = [("int8", "int8", (15, 16, 17, 31, 33, 127, 764, 772, 1001)),
+           ("float16", "float16", (7, 8, 9, 15, 17, 63, 501)),
+           ("float32", "float32", (5, 31, 32, 33, 63, 191, 193, 1001)), ("float32", "float16", (7, 8, 9, 11, 33, 1001)),
            ("float16", "float32", (3, 9, 33, 501))]
 
 
@@ -253,8 +254,8 @@ def test_row_gathers_on_the_gpu(src, dst, widths):
     torch = pytest.importorskip("torch")
     rng = np.random.default_rng(len(widths))
     with P.Context(0) as ctx:
-        for d in widths:
-            rows, count = 211, 333
+        # selections of more and of fewer rows than the table has
+        for d, rows, count in [(d, rows, 333) for d in widths for rows in (211, 401)]:
             x = _source((rows, d), src, rng)
             idx = rng.integers(0, rows, count).astype("<i8")
             idx[:2] = (rows - 1, 0)
