@@ -33,16 +33,21 @@ def _chains(shape, axis, rng):
             ("int8", [EN.Dequantize(sc(), zero_point=zp, axis=axis)]),
             ("int8", [EN.Dequantize(sc(), axis=axis), EN.Cast("float16")]),
             ("float32", [EN.Quantize(sc(), axis=axis)]),
-            ("float16", [EN.Cast("float32", "exact"), EN.Quantize(sc(), axis=axis)])]
+            ("float16", [EN.Cast("float32", "exact"), EN.Quantize(sc(), axis=axis)]),
+            # bf16 sources, and chains without a compile-time kernel body
+            ("bfloat16", [EN.Cast("float32", "exact")]),
+            ("int8", [EN.Dequantize(sc(), zero_point=zp, axis=axis), EN.Cast("bfloat16")]),
+            ("bfloat16", [EN.Cast("float32", "exact"), EN.Quantize(sc(), axis=axis)])]
 
 
 def _source(shape, dtype, rng):
     if dtype == "int8":
         return rng.integers(-128, 128, shape, dtype=np.int8)
-    x = (rng.standard_normal(shape) * 3).astype(dtype)
-    x.reshape(-1)[:: 97] = np.resize(np.array([np.nan, np.inf, -np.inf, -0.0, 6e4, 1e-7], dtype),
+    narrow = "float32" if dtype == "bfloat16" else dtype
+    x = (rng.standard_normal(shape) * 3).astype(narrow)
+    x.reshape(-1)[:: 97] = np.resize(np.array([np.nan, np.inf, -np.inf, -0.0, 6e4, 1e-7], narrow),
                                      x.reshape(-1)[::97].size)
-    return x
+    return (x.view(np.uint32) >> 16).astype(np.uint16) if dtype == "bfloat16" else x
 
 
 # (rows, cols) [batch] around the tile widths: one row of a vector less or
@@ -378,3 +383,38 @@ def test_large_tiles_on_the_gpu(case):
         torch.cuda.synchronize()
     assert torch.equal(buf[GUARD:-GUARD], want)
     assert bool((buf[:GUARD] == 0xA5).all()) and bool((buf[-GUARD:] == 0xA5).all())
+
+
+# One case per kernel that takes buffers at any address, and one per kernel
+# whose launches then run element-wise
+SHIFTED = [("transpose", (3, 33, 67), transpose_cases), ("transpose", (None, 6, 640), transpose_cases),
+           ("rows", ROWS[2], rows_cases), ("rows", ROWS[6], rows_cases), ("image", IMAGES[1], image_cases),
+           ("image", IMAGES[2], image_cases), ("flat", (50, 21), flat_cases), ("flat", (37, 16), flat_cases),
+           ("permute", (2, 5, 12, 64), permute_cases), ("element", ELEMENTS[0], element_cases)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("group", SHIFTED, ids=["%s %s" % (k, c) for k, c, _ in SHIFTED])
+def test_shifted_buffers_on_the_gpu(group):
+    """Device-resident sources and results that start one element, and one
+    byte, past a 64-byte boundary: the same bytes, and none around them."""
+    torch = pytest.importorskip("torch")
+    _, case, make = group
+    with P.Context(0) as ctx:
+        for name, blob, x in make(case):
+            print("[gpu-case]", name, flush=True)
+            want = _want(blob, x)
+            n = len(want)
+            b = P.Bound(P.Plan(blob), {}, {})
+            src = torch.from_numpy(np.ascontiguousarray(x).view(np.uint8).reshape(-1).copy()).cuda()
+            for s_at, d_at in ((x.itemsize, b.element_size), (1, 1), (0, 1), (1, 0)):
+                dev = torch.full((src.numel() + 2 * GUARD,), 0x5A, dtype=torch.uint8, device="cuda")
+                dev[GUARD + s_at:GUARD + s_at + src.numel()].copy_(src)
+                buf = torch.full((n + 2 * GUARD,), 0xA5, dtype=torch.uint8, device="cuda")
+                at = GUARD + d_at
+                ctx.relayout_device(b, dev.data_ptr() + GUARD + s_at, buf.data_ptr() + at,
+                                    stream=torch.cuda.current_stream().cuda_stream)
+                torch.cuda.synchronize()
+                got = buf.cpu().numpy()
+                assert got[at:at + n].tobytes() == want, (name, s_at, d_at)
+                assert (got[:at] == 0xA5).all() and (got[at + n:] == 0xA5).all(), (name, s_at, d_at)
